@@ -293,6 +293,11 @@ struct AttnArgs {
   // (tag << 32 | value bits) at ocells + h * head_dim instead of stored
   const unsigned long long *epoch;
   unsigned long long *ocells;
+  // pbx_qkvr_attn_o_*: contexts of more than split_at positions (0: none)
+  // are split over the workgroups of a KV group, whose partial states travel
+  // as cells [n_heads][parts][PBX_PS_CELLS]
+  unsigned long long *pcells;
+  int split_at;
 };
 
 // One workgroup per query head (llama.js:258-301 / llama-streaming.js:543-573):
@@ -768,6 +773,237 @@ __device__ __forceinline__ float poll_cell(const unsigned long long *cp, unsigne
   return __builtin_nanf("");
 }
 
+// Long contexts in the fused launch: the 16 workgroups of four query heads of
+// one KV group (4 heads x 4 parts) take every 16th slot of 32 positions each,
+// for all four heads, instead of each repeating its head's whole context: K
+// and V leave the XCD's L2 once instead of 16 times.  A workgroup's state of
+// a head (weighted V sum, its maximum and sum) is published as cells tagged
+// like the q|k|v rows, and every workgroup then merges the 16 states of its
+// own head and goes on to its o rows.  All the workgroups must be resident
+// at once (the host checks the grid against the CUs); the waits are bounded.
+// Bound by the K/V transfer and by the hand-off's ~2 us: Llama-1B decode at KV
+// 3500 888 -> 403 us a token, 2000: 543 -> 371, 1000: 406 -> 361.  The hand-off
+// costs more than it saves on short contexts (700: 374 unsplit against 363, 512:
+// 350 against 359, 128: 323 against 354), so split_at is 640.
+#define PBX_PS_HEADS 4
+#define PBX_PS_CELLS 66  // 64 dims, maximum, sum
+#define PBX_PS_SLOTS 8   // slots in flight
+
+// J slots p + 16 j0 .. of the workgroup, folded into the four heads' states.
+template <int J, class Ready>
+__device__ __forceinline__ void split_chunk(const float *kb, const float *vb, int kvdim, int dcol,
+                                            int s0, int stride, int pl, int nc, Ready &&ready,
+                                            const float4 (&qq)[PBX_PS_HEADS], const float4 &kn,
+                                            const float4 &vn, float (&m)[PBX_PS_HEADS],
+                                            float (&l)[PBX_PS_HEADS],
+                                            float4 (&acc)[PBX_PS_HEADS]) {
+  float4 k[J], v[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    k[j] = *reinterpret_cast<const float4 *>(
+        kb + (size_t)min(32 * (s0 + stride * j) + pl, nc - 1) * kvdim + dcol);
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    v[j] = *reinterpret_cast<const float4 *>(
+        vb + (size_t)min(32 * (s0 + stride * j) + pl, nc - 1) * kvdim + dcol);
+  ready();
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (32 * (s0 + stride * j) + pl == nc - 1) {
+      k[j] = kn;
+      v[j] = vn;
+    }
+#pragma unroll
+  for (int i = 0; i < PBX_PS_HEADS; ++i) {
+    float s[J];
+    float mc = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const float d = wave_sum<8>(
+          fmaf(qq[i].x, k[j].x, fmaf(qq[i].y, k[j].y, fmaf(qq[i].z, k[j].z, qq[i].w * k[j].w))));
+      s[j] = 32 * (s0 + stride * j) + pl < nc ? d : -INFINITY;
+      mc = fmaxf(mc, s[j]);
+    }
+    const float mn = fmaxf(m[i], mc);
+    const float ms = mn == -INFINITY ? 0.f : mn;  // a row with no position yet
+    const float f = __builtin_amdgcn_exp2f(m[i] - ms);
+    float ls = 0.f;
+    float4 a = make_float4(acc[i].x * f, acc[i].y * f, acc[i].z * f, acc[i].w * f);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const float p = __builtin_amdgcn_exp2f(s[j] - ms);
+      ls += p;
+      a.x = fmaf(p, v[j].x, a.x);
+      a.y = fmaf(p, v[j].y, a.y);
+      a.z = fmaf(p, v[j].z, a.z);
+      a.w = fmaf(p, v[j].w, a.w);
+    }
+    l[i] = fmaf(l[i], f, ls);
+    acc[i] = a;
+    m[i] = mn;
+  }
+}
+
+// Leaves the states of query head h in st_m / st_l / st_acc (wave w holds the
+// merged states w and w + 8 of the head's `parts` <= 16 states).
+__device__ __forceinline__ void attention_split_states(const AttnArgs &a, const int h,
+                                                       const int part, const int parts,
+                                                       const int nc, const unsigned tag,
+                                                       float *st_m, float *st_l,
+                                                       float (*st_acc)[PBX_HA_MAX_HD]) {
+  constexpr int HG = PBX_PS_HEADS, HD = PBX_HA_MAX_HD, NW = PBX_HA_WAVES;
+  __shared__ __attribute__((aligned(16))) float rows[HG + 2][HD];  // q of the heads, new k, v
+  __shared__ float ps_m[HG][NW], ps_l[HG][NW];
+  __shared__ __attribute__((aligned(16))) float ps_acc[HG][NW][HD];
+  const int Gq = a.n_heads / a.n_kv_heads, g = h / Gq, kvdim = a.n_kv_heads * HD;
+  const int h0 = h - h % HG, p = h % HG + HG * part, P = HG * parts;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int dg = lane & 15, dcol = 4 * dg, pl = 4 * w + (lane >> 4);
+  const float *kb = a.kcache + (size_t)g * HD, *vb = a.vcache + (size_t)g * HD;
+  const int spin = a.spin > 0 ? a.spin : PBX_CELL_SPIN;
+  const unsigned ptag = tag - (unsigned)a.skew;  // published with the launch's own tag
+
+  float m[HG], l[HG];
+  float4 acc[HG], qq[HG], kn = make_float4(0.f, 0.f, 0.f, 0.f), vn = kn;
+#pragma unroll
+  for (int i = 0; i < HG; ++i) {
+    m[i] = -INFINITY;
+    l[i] = 0.f;
+    acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    qq[i] = acc[i];
+  }
+  const int ns = (nc + 31) / 32;
+  const bool newest = (ns - 1) % P == p;
+  auto ready = [&]() {
+    if (w < HG || (w < HG + 2 && newest))
+      rows[w][lane] = poll_cell(
+          a.cells + (w < HG ? (h0 + w) * HD : a.qdim + (w - HG) * kvdim + g * HD) + lane, tag, spin,
+          a.status);
+    lds_barrier();
+    const float c = a.scale * 1.44269504088896340736f;  // scale * log2 e
+#pragma unroll
+    for (int i = 0; i < HG; ++i) {
+      const float4 t = *reinterpret_cast<const float4 *>(&rows[i][dcol]);
+      qq[i] = make_float4(t.x * c, t.y * c, t.z * c, t.w * c);
+    }
+    if (newest) {
+      kn = *reinterpret_cast<const float4 *>(&rows[HG][dcol]);
+      vn = *reinterpret_cast<const float4 *>(&rows[HG + 1][dcol]);
+    }
+  };
+  auto none = [] {};
+  bool first = true;
+  for (int s0 = p; s0 < ns;) {
+    const int J = min(PBX_PS_SLOTS, (ns - s0 + P - 1) / P);
+    switch (J) {
+#define PBX_SPLIT_CHUNK(n)                                                                \
+  case n:                                                                                 \
+    if (first)                                                                            \
+      split_chunk<n>(kb, vb, kvdim, dcol, s0, P, pl, nc, ready, qq, kn, vn, m, l, acc);   \
+    else                                                                                  \
+      split_chunk<n>(kb, vb, kvdim, dcol, s0, P, pl, nc, none, qq, kn, vn, m, l, acc);    \
+    break;
+      PBX_SPLIT_CHUNK(1) PBX_SPLIT_CHUNK(2) PBX_SPLIT_CHUNK(3) PBX_SPLIT_CHUNK(4)
+      PBX_SPLIT_CHUNK(5) PBX_SPLIT_CHUNK(6) PBX_SPLIT_CHUNK(7) PBX_SPLIT_CHUNK(8)
+#undef PBX_SPLIT_CHUNK
+      default: break;
+    }
+    first = false;
+    s0 += J * P;
+  }
+
+  // the wave's 4 rows, then the 8 waves (wave i < HG: head i), then publish
+#pragma unroll
+  for (int i = 0; i < HG; ++i) {
+    const float mw = pair_max<32>(pair_max<16>(m[i]));
+    const float er = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[i] - mw);
+    const float lw = pair_sum<32>(pair_sum<16>(l[i] * er));
+    const float4 aw = make_float4(pair_sum<32>(pair_sum<16>(acc[i].x * er)),
+                                  pair_sum<32>(pair_sum<16>(acc[i].y * er)),
+                                  pair_sum<32>(pair_sum<16>(acc[i].z * er)),
+                                  pair_sum<32>(pair_sum<16>(acc[i].w * er)));
+    if (lane == 0) {
+      ps_m[i][w] = mw;
+      ps_l[i][w] = lw;
+    }
+    if (lane < 16) *reinterpret_cast<float4 *>(&ps_acc[i][w][dcol]) = aw;
+  }
+  lds_barrier();
+  if (w < HG) {
+    float M = -INFINITY, den = 0.f, num = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) M = fmaxf(M, ps_m[w][i]);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const float mi = ps_m[w][i];
+      const float e = mi == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mi - M);
+      den = fmaf(e, ps_l[w][i], den);
+      num = fmaf(e, ps_acc[w][i][lane], num);
+    }
+    unsigned long long *cp = a.pcells + ((size_t)(h0 + w) * P + p) * PBX_PS_CELLS;
+    const unsigned long long th = (unsigned long long)ptag << 32;
+    __hip_atomic_store(cp + lane, th | __float_as_uint(num), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    if (lane < 2)
+      __hip_atomic_store(cp + HD + lane, th | __float_as_uint(lane ? den : M), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+
+  // states w and w + 8 of head h: four cells a lane polled together (lane:
+  // the dim's sums; lanes 0 and 1 of the second pair: maximum and sum)
+  const unsigned long long *hp = a.pcells + (size_t)h * P * PBX_PS_CELLS;
+  const unsigned long long *cp[4];
+  bool use[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int st = w + NW * (i & 1);
+    use[i] = st < P && (i < 2 || lane < 2);
+    cp[i] = hp + (size_t)(st < P ? st : 0) * PBX_PS_CELLS + (i < 2 ? lane : HD + (lane & 1));
+  }
+  unsigned long long v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    v[i] = use[i] ? __hip_atomic_load(cp[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                  : (unsigned long long)ptag << 32;
+  auto missing = [&]() {
+    return (unsigned)(v[0] >> 32) != ptag || (unsigned)(v[1] >> 32) != ptag ||
+           (unsigned)(v[2] >> 32) != ptag || (unsigned)(v[3] >> 32) != ptag;
+  };
+  for (int it = 0; missing() && it < spin; ++it) {
+    __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if ((unsigned)(v[i] >> 32) != ptag)
+        v[i] = __hip_atomic_load(cp[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (missing())
+    __hip_atomic_fetch_or(a.status, PBX_DEV_WAIT_TIMEOUT, __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_AGENT);
+  float f[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    f[i] = (unsigned)(v[i] >> 32) == ptag ? __uint_as_float((unsigned)v[i]) : __builtin_nanf("");
+  float mw = -INFINITY, lw = 0.f, aw = 0.f, M[2], D[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    M[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[2 + i]), 0));
+    D[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[2 + i]), 1));
+    if (w + NW * i >= P) M[i] = -INFINITY;
+    mw = fmaxf(mw, M[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float e = M[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M[i] - mw);
+    lw = fmaf(e, D[i], lw);
+    aw = fmaf(e, f[i], aw);
+  }
+  if (lane == 0) {
+    st_m[w] = mw;
+    st_l[w] = lw;
+  }
+  st_acc[w][lane] = aw;
+}
+
 // MAXJ: position slots a wave keeps in flight (16 slots of K and V are
 // 128 registers a lane; a caller with less room passes fewer).
 template <bool SPEC, int IPT = 0, bool FUSED = false, int MAXJ = 16>
@@ -825,6 +1061,7 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   int s0 = 0;
   unsigned tag = 0;
+  bool split = false;
   if constexpr (FUSED) {
     tag = cell_tag(a.epoch ? *a.epoch : a.cells[a.cell_n]) + (unsigned)a.skew;
     const int spin = a.spin > 0 ? a.spin : PBX_CELL_SPIN;
@@ -847,7 +1084,8 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
     };
     auto none = [] {};
     bool first = true;
-    while (32 * s0 < nc) {
+    if constexpr (IPT > 0) split = a.split_at > 0 && nc > a.split_at;
+    while (!split && 32 * s0 < nc) {
       const int J = min(MAXJ, (nc - 32 * s0 + 31) / 32);
       switch (J) {
 #define PBX_HEAD_CHUNK_N(n)                                                                \
@@ -888,20 +1126,26 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
     s0 += J;
   }
 
-  // merge in two levels: the wave's 4 rows (same dims, 16 lanes apart) in
-  // registers, then the 8 wave states through LDS in one wave
-  const float mw = pair_max<32>(pair_max<16>(m));  // finite for wave 0 (position 0)
-  const float er = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mw);
-  const float lw = pair_sum<32>(pair_sum<16>(l * er));
-  const float4 aw = make_float4(pair_sum<32>(pair_sum<16>(acc.x * er)),
-                                pair_sum<32>(pair_sum<16>(acc.y * er)),
-                                pair_sum<32>(pair_sum<16>(acc.z * er)),
-                                pair_sum<32>(pair_sum<16>(acc.w * er)));
-  if (lane == 0) {
-    st_m[w] = mw;
-    st_l[w] = lw;
+  if constexpr (FUSED && IPT > 0) {
+    if (split)
+      attention_split_states(a, h, part, a.n_heads * hd / (256 * IPT), nc, tag, st_m, st_l, st_acc);
   }
-  if (lane < 16) *reinterpret_cast<float4 *>(&st_acc[w][4 * dg]) = aw;
+  if (!split) {
+    // merge in two levels: the wave's 4 rows (same dims, 16 lanes apart) in
+    // registers, then the 8 wave states through LDS in one wave
+    const float mw = pair_max<32>(pair_max<16>(m));  // finite for wave 0 (position 0)
+    const float er = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mw);
+    const float lw = pair_sum<32>(pair_sum<16>(l * er));
+    const float4 aw = make_float4(pair_sum<32>(pair_sum<16>(acc.x * er)),
+                                  pair_sum<32>(pair_sum<16>(acc.y * er)),
+                                  pair_sum<32>(pair_sum<16>(acc.z * er)),
+                                  pair_sum<32>(pair_sum<16>(acc.w * er)));
+    if (lane == 0) {
+      st_m[w] = mw;
+      st_l[w] = lw;
+    }
+    if (lane < 16) *reinterpret_cast<float4 *>(&st_acc[w][4 * dg]) = aw;
+  }
   lds_barrier();
   if (w == 0) {
     const float mi = lane < PBX_HA_WAVES ? st_m[lane] : -INFINITY;

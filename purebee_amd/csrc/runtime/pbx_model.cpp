@@ -49,6 +49,10 @@ struct AttnArgsHost {  // AttnArgs in pbx_decode.hip
   // the small-model step: the tag's epoch and the published head outputs
   const unsigned long long *epoch = nullptr;
   unsigned long long *ocells = nullptr;
+  // pbx_qkvr_attn_o_*: cells of the partial states and the context length
+  // above which the positions are split over a KV group's workgroups
+  unsigned long long *pcells = nullptr;
+  int split_at = 0;
 };
 
 struct AttnSplitArgsHost {  // AttnSplitArgs in pbx_decode.hip
@@ -228,6 +232,9 @@ struct pbx_model {
   // layer's epoch ((qkv_rows + 64) cells, allocated with the first step)
   bool qkv_attn = true;
   unsigned long long *qa_cells = nullptr;
+  // context length above which the joined launch splits the positions over
+  // the workgroups of a KV group (PBX_ATTN_SPLIT at creation; 0: never)
+  int attn_split = 640;
   // state[0] position, [1] token, [2] step, [3] status word (bits set by
   // device-side waits that gave up; read and cleared by the host calls)
   int *state = nullptr;
@@ -704,10 +711,18 @@ static int build_ops(pbx_model *m) {
   // (pbx_qkvr_attn_o_r<RT>c<IPT>: IPT 1 with 16-row GEMV tiles, IPT 2 with
   // 32-row tiles).
   hipFunction_t fqa = nullptr;
-  const size_t cell_stride = (size_t)m->qkv_rows + 64;
+  size_t cell_stride = (size_t)m->qkv_rows + 64;
   const int qa_rows = o_ipt == 2 ? 32 : 16;
   const std::string qa_name = o_ipt == 2 ? "pbx_qkvr_attn_o_r8c2" : "pbx_qkvr_attn_o_r4c1";
   if ((o_ipt == 1 || o_ipt == 2) && qa_fit) fqa = pbx_kernel_by_name(c, qa_name);
+  // Long contexts: the positions split over the 16 workgroups of four heads
+  // of a KV group, which wait for each other's states, so the whole grid (one
+  // workgroup a CU) must fit the CUs.
+  const int parts = o_ipt ? g.dim / (256 * o_ipt) : 0;
+  const bool qa_split = fqa && m->attn_split > 0 && g.n_heads / g.n_kv_heads % 4 == 0 &&
+                        4 * parts <= 16 &&
+                        m->qkv_rows / qa_rows + g.n_heads * parts <= c->cu_count;
+  if (qa_split) cell_stride += (size_t)g.n_heads * 4 * parts * 66;
   if (fqa && !m->qa_cells) {
     const size_t cb = (size_t)g.n_layers * cell_stride * 8;
     int rc = dalloc(m, (void **)&m->qa_cells, cb);
@@ -797,6 +812,10 @@ static int build_ops(pbx_model *m) {
         a.attn.cell_n = m->qkv_rows;
         a.attn.qdim = g.dim;
         a.attn.status = m->state + 3;
+        if (qa_split) {
+          a.attn.pcells = cells + m->qkv_rows + 64;
+          a.attn.split_at = m->attn_split;
+        }
         if (l == m->test_layer) {
           a.attn.skew = m->test_skew;
           a.attn.spin = m->test_spin;
@@ -1348,6 +1367,7 @@ extern "C" int pbx_model_create(pbx_ctx *c, const pbx_model_config *cfg, pbx_mod
   m->attn_mode = attention_mode(g);
   if (const char *e = getenv("PBX_QKV_ATTN")) m->qkv_attn = e[0] != '0';
   if (const char *e = getenv("PBX_ATTN_O")) m->attn_o_ipt = atoi(e);
+  if (const char *e = getenv("PBX_ATTN_SPLIT")) m->attn_split = std::max(0, atoi(e));
   if (const char *e = getenv("PBX_GRAPH_STEPS")) m->graph_steps = atoi(e);
   if (const char *e = getenv("PBX_FFN")) m->ffn_join = e[0] != '0';
   if (const char *e = getenv("PBX_SMALL_STEP")) m->small_ok = e[0] != '0';

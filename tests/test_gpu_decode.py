@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 # Switches that select other decode kernels at model creation; the tests
 # that check which kernels a step launches clear them first, so they hold
 # whatever the caller's environment selects.
-PATH_SWITCHES = ("PBX_FFN", "PBX_QKV_ATTN", "PBX_ATTN_O", "PBX_GEMV_INT", "PBX_SMALL_STEP")
+PATH_SWITCHES = ("PBX_FFN", "PBX_QKV_ATTN", "PBX_ATTN_O", "PBX_GEMV_INT", "PBX_SMALL_STEP",
+                 "PBX_ATTN_SPLIT")
 
 
 @pytest.fixture
@@ -274,6 +275,39 @@ def test_fused_qkv_attention_long_context(ctx, default_paths):
     assert list(ga) == list(gb)
     fused.free()
     plain.free()
+
+
+@pytest.mark.parametrize("kv_heads", [8, 4])
+@pytest.mark.parametrize("n", [1, 31, 510, 4094])
+def test_split_context_attention(ctx, default_paths, kv_heads, n):
+    """The joined launch with the context split over the 16 workgroups of four
+    heads (PBX_ATTN_SPLIT=1: from two positions on; the default leaves short
+    contexts whole) against the same launch unsplit, in a 1-layer model, for
+    three steps from position n: a slot's edges (32 positions), a workgroup's
+    first slot only, the 16-slot stride (512), and the second chunk of 8 slots
+    a workgroup (16 * 8 * 32 = 4096).  Both sum the same fp32 products in
+    another order: some 1e-6 of the O(1) logits, 1e-4 as for the other paths.
+    Then 13 greedy steps through the step graphs."""
+    monkeypatch = default_paths
+    print(f"[case] split context, {kv_heads} KV heads, positions {n}..", flush=True)
+    cfg = tiny(TYPE_Q4_0, TYPE_Q4_0, dim=2048, hidden_dim=8192, n_layers=1, n_heads=32,
+               n_kv_heads=kv_heads, vocab_size=512, max_seq=4128)
+    toks = [int(t) for t in synth.random_tokens(132, n + 3, cfg["vocab_size"])]
+    out = {}
+    for split in ("0", "1"):
+        monkeypatch.setenv("PBX_ATTN_SPLIT", split)
+        model = synth.build(ctx, cfg, 131)
+        model.forward(toks[:n], 0, want_logits=False)
+        steps = [model.forward([toks[p]], p)[0] for p in range(n, n + 3)]
+        kern = {k for _, k, _, _ in model.profile(toks[-1], n + 2, 1)}
+        assert "pbx_qkvr_attn_o_r8c2" in kern
+        out[split] = steps, list(model.generate(toks[-1], n + 2, 13))
+        model.free()
+    worst = max(float(np.abs(a - b).max()) for a, b in zip(out["0"][0], out["1"][0]))
+    print(f"  max-abs {worst:.2e}; greedy {out['0'][1]} / {out['1'][1]}")
+    assert all(np.isfinite(a).all() for a in out["1"][0])
+    assert worst <= 1e-4
+    assert out["0"][1] == out["1"][1]
 
 
 def test_non_finite_activation_propagates(ctx):
