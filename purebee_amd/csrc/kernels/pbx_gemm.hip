@@ -41,14 +41,15 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 struct GemmArgs {
   const uint8_t *qs;      // weight plane
   const uint16_t *dsc;    // fp16 scale plane (4-row groups)
-  const _Float16 *X16;    // [Mpad][K] scaled fp16 activations
-  const _Float16 *X16lo;  // [Mpad][K] rounding residual of X16
+  const _Float16 *X16;    // [K / 32][Mpad][32] scaled fp16 activations
+  const _Float16 *X16lo;  // [K / 32][Mpad][32] rounding residual of X16
   const float *inv;       // [Mpad] power of two undoing the row scale
   const float *bias;      // [N] or null (single split only)
   float *Y;               // KS == 1: [M][N]; else partials [KS][M][N]
   int M, N, Npad, B, KS;
   int accumulate;         // 1: Y[m][n] += result (residual), single split only
   const uint16_t *msc;    // Q4_1 fp16 min plane
+  int Mpad;               // rows of a block of X16 (M padded to the kernel's M tile)
 };
 
 namespace {
@@ -172,7 +173,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
   const int li = lane & 15, g = lane >> 4;
   const int n0 = (blockIdx.x * 4 + wave) * (16 * NT);
   const int m0 = blockIdx.y * (16 * MT);
-  const int K = a.B * 32;
   const int per = (a.B + a.KS - 1) / a.KS;
   const int b0 = blockIdx.z * per;
   const int b1 = min(a.B, b0 + per);
@@ -197,7 +197,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
           load_codes<TYPE>(a, n0 + 16 * u + li, bb, g, &raw[j][u], &dbits[j][u], &mbits[j][u]);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-          const size_t off = (size_t)(m0 + 16 * t + li) * K + bb * 32 + 8 * g;
+          const size_t off = ((size_t)bb * a.Mpad + m0 + 16 * t + li) * 32 + 8 * g;
           A[j][t] = *reinterpret_cast<const half8 *>(a.X16 + off);
           Alo[j][t] = *reinterpret_cast<const half8 *>(a.X16lo + off);
         }
@@ -281,20 +281,21 @@ GEMM_KERNEL(pbx_gemm_f16_m2_n2, PBX_F16, 2, 2)
 // 8h..8h+7 (a lane reads its 8 code bytes once), the Q8_0 bytes 8h.. and
 // 16+8h.., the F16 halves likewise.  Each lane's 16 outputs share one column
 // (weight row), so the block scale is one value per lane.
-// Workgroup tile MT (M, 128 or 64) x 128 (N), four waves in 2 x 2, wave tile
-// MT / 2 x 64 (MT / 64 x 2 MFMA tiles).  A ring of NS LDS stages, each
-// [hi/lo][MT rows][4 chunks of 8 halves] of activations, the 128 weight rows'
-// code bytes (or F16 weights) and their scales (and Q4_1 mins).  Per block
-// every wave issues the same number of DMA instructions (global_load_lds:
-// lane i's bytes land at the instruction's LDS base + size * i): MT / 32
-// activation chunks and its share of the weight data (DmaW), so one wait
-// count fits every wave;
-// the loads are issued from inline assembly with SGPR bases, so
-// the compiler adds no waits of its own, and no register load is in flight
-// across the block loop.  The chunks of activation row r are stored in the
-// order q ^ swz(r), swz(r) = ((r >> 1) ^ (r >> 3)) & 3: the 16-byte reads of
-// 16 consecutive rows at one chunk fall in 16 distinct bank groups.  The
-// loop is unrolled by NS so every LDS offset is an immediate.
+// The activations are block-major (X16: [K / 32][Mpad][32]): a tile's block is
+// contiguous, where rows K apart put all its 64-byte pieces on few L2
+// channels and read half lines (16384 x 2048 at 2000 rows: 364 -> 321 us with
+// that alone; 2048 x 8192 at 512 71 -> 65).  The chunks of activation row r
+// are stored in the order q ^ swz(r), swz(r) = ((r >> 1) ^ (r >> 3)) & 3: the
+// 16-byte reads of 16 consecutive rows at one chunk fall in 16 distinct bank
+// groups.  Everything reaches LDS by DMA (global_load_lds: lane i's bytes land
+// at the instruction's LDS base + size * i), issued from inline assembly with
+// SGPR bases, so the compiler adds no waits of its own; every wave issues the
+// same number of DMA instructions per block, so one wait count fits all, and
+// no register load is in flight across the block loop.
+// Two kernels: gemm_dma (128 x 128 tiles, pipelined over registers, two
+// workgroups a CU) and gemm_dma64 (64 x 128, four to five a CU, which hide the
+// latencies of one block for each other; the pipelined form took 57 -> 63 us
+// of 8192 x 2048 at 512 rows and 0.5-1.5 us more at few blocks).
 // Needs X16 / X16lo padded to a multiple of 128 rows.
 // ---------------------------------------------------------------------------
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -323,13 +324,59 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Weight bytes of one row and block in the stage: Q4_0 / Q4_1 16 code bytes,
-// Q8_0 32, F16 64 (the fp16 weights); per-block scales (and Q4_1 mins) follow.
+// Stores of a wave's TT x 2 tiles of 32 x 32 outputs at rows mw.. and columns
+// n0.. (SW: silu(gate) * up).
+template <bool SW, int TT>
+__device__ __forceinline__ void store_tiles(const GemmArgs &a, const floatx16 (&acc)[TT][2], int mw,
+                                            int n0, int wn, int lr, int h) {
+  if constexpr (SW) {
+    const int NO = a.N / 2, c = blockIdx.x * 64 + 32 * wn + lr;  // the lane's hidden column
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = mw + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (m < a.M) {
+          const float iv = a.inv[m];
+          a.Y[(size_t)m * NO + c] = silu(acc[t][0][r] * iv) * (acc[t][1][r] * iv);
+        }
+      }
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int n = n0 + 32 * u + lr;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = mw + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (m < a.M && n < a.N) {
+          const float v = acc[t][u][r] * a.inv[m];
+          if (a.KS == 1) {
+            float *y = a.Y + (size_t)m * a.N + n;
+            if (a.accumulate)
+              *y += v;
+            else
+              *y = v + (a.bias ? a.bias[n] : 0.f);
+          } else {
+            a.Y[((size_t)blockIdx.z * a.M + m) * a.N + n] = v;
+          }
+        }
+      }
+    }
+}
+
+// A weight group: 64 bytes of every row, i.e. SB consecutive blocks (Q4_0 /
+// Q4_1 four of 16 code bytes, Q8_0 two of 32, F16 one of 64), and their
+// scales (and Q4_1 mins) as in the planes, [32 four-row groups][SB][4].
 template <int TYPE> struct DmaW {
   static constexpr int CB = TYPE == PBX_F16 ? 64 : TYPE == PBX_Q8 ? 32 : 16;
-  static constexpr int CODES = 128 * CB;                  // bytes of a stage
-  static constexpr int NSC = TYPE == PBX_F16 ? 0 : TYPE == PBX_Q41 ? 2 : 1;  // 256-byte planes
-  static constexpr int WD = TYPE == PBX_Q8 || TYPE == PBX_F16 ? 2 : 1;      // weight DMAs a wave
+  static constexpr int SB = 64 / CB;
+  static constexpr int CODES = 128 * 64;
+  static constexpr int NSC = TYPE == PBX_F16 ? 0 : TYPE == PBX_Q41 ? 2 : 1;
+  static constexpr int PLANE = 128 * SB * 2;
+  static constexpr int BYTES = CODES + NSC * PLANE;
 };
 
 // SW: the gate|up weight of a Llama FFN (N / 2 gate rows, then N / 2 up
@@ -339,10 +386,344 @@ template <int TYPE> struct DmaW {
 // wave's two 32-column subtiles (u = 0, 1) hold a gate and its up for one
 // lane's column; Y is [M][N / 2].  Needs N / 2 a multiple of 64 and no K
 // split.
-template <int TYPE, int NS, int MT = 128, bool SW = false>
+// 128 x 128 tiles, four waves in 2 x 2, wave tile 64 x 64.  Rings of three
+// activation stages [hi/lo][128 rows][4 chunks] and of three weight groups: a
+// group's 64 bytes of a row are one request, where one block's 16 would fetch
+// its line four times.  16384 x 2048 Q4_0 at 2000 rows: 312 us = 430 TFLOP/s
+// useful, 860 of MFMA work (355-370 before; MFMAs alone, their operands
+// constant, 205); F16 8192 x 2048 at 512 60 -> 54 us.  What is left is LDS
+// traffic (36 KB read and 18.7 written a block), 108 vector operations to 16
+// MFMAs, and the clock under both.
+template <int TYPE, bool SW = false>
 __device__ __forceinline__ void gemm_dma(const GemmArgs &a) {
-  static_assert(MT == 128 || MT == 64, "M tile");
+  constexpr int MT = 128;
   typedef DmaW<TYPE> W;
+  constexpr int NA = MT / 64;                 // activation chunks a wave and plane
+  constexpr int TT = MT / 64;                 // 32-row MFMA tiles a wave
+  constexpr int PS = MT * 32 * 2;             // bytes of a stage's hi (or lo) plane
+  constexpr int STAGE = 2 * PS;               // bytes
+  constexpr int SB = W::SB;
+  constexpr int WOFF = 3 * STAGE;             // the ring of three weight groups
+  __shared__ __attribute__((aligned(1024))) uint8_t S[3 * (STAGE + W::BYTES)];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: SGPR bases
+  const int lr = lane & 31, h = lane >> 5;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int n0 = blockIdx.x * 128 + wn * 64;
+  const int mblk = blockIdx.y * MT;
+  const int m0 = wm * (MT / 2);
+  const int per = (a.B + a.KS - 1) / a.KS;
+  const int b0 = blockIdx.z * per;
+  const int b1 = min(a.B, b0 + per);
+  const floatx16 zero16 = {};
+
+  floatx16 acc[TT][2];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) acc[t][u] = zero16;
+
+  if (b0 < b1) {
+    // Activation DMA i (i < NA) of this wave and plane: LDS chunks
+    // (4 i + wave) * 64 + lane, one KB that is contiguous in X16 too.
+    unsigned avoff[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const int c = (4 * i + wave) * 64 + lane;
+      const int r = c >> 2, q = (c & 3) ^ a_swz(r);
+      avoff[i] = (unsigned)((r * 32 + q * 8) * 2);
+    }
+    const size_t xstep = (size_t)a.Mpad * 64;  // bytes of a block
+    const uint8_t *xhi = reinterpret_cast<const uint8_t *>(a.X16) + (size_t)mblk * 64;
+    const uint8_t *xlo = reinterpret_cast<const uint8_t *>(a.X16lo) + (size_t)mblk * 64;
+    const unsigned lbase = lds_addr(&S[0]);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane(lbase + wave * 1024);
+    auto dma_x = [&](int b, int slot) {
+      const unsigned so = slot * STAGE;
+      const size_t xo = b * xstep;
+#pragma unroll
+      for (int i = 0; i < NA; ++i) dma_to_lds_s<16>(xhi + xo, avoff[i], lds0 + so + 4096 * i);
+#pragma unroll
+      for (int i = 0; i < NA; ++i) dma_to_lds_s<16>(xlo + xo, avoff[i], lds0 + so + PS + 4096 * i);
+    };
+    // Weight DMAs of this wave for the group of blocks gb .. gb + SB - 1
+    // (bases at the workgroup's first row, so the per-lane offsets stay
+    // small): code DMAs k = 0, 1 of 16 rows each, row 16 (2 wave + k) +
+    // lane / 4, whose four chunks are stored in the order q ^ swz(row) like
+    // the activations'; plane DMAs of one dword a lane.  Chunks and dwords
+    // past the row's last block are clamped to it (never used).
+    const size_t rowbytes = (size_t)a.B * W::CB;
+    // SW: the weight row of tile row i (the gate or up rows of the
+    // workgroup's hidden columns; relative to row 0)
+    auto sw_row = [&](int i) -> int {
+      const int c = i >> 5;
+      return ((c & 1) ? a.N / 2 : 0) + blockIdx.x * 64 + 32 * (c >> 1) + (i & 31);
+    };
+    const uint8_t *cbase = a.qs + (SW ? 0 : (size_t)blockIdx.x * 128 * rowbytes);
+    unsigned crow[2];
+    unsigned cq[2];
+    const unsigned clast = (unsigned)rowbytes - 16;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int i = 16 * (2 * wave + k) + (lane >> 2);
+      cq[k] = (unsigned)((lane & 3) ^ a_swz(i)) * 16;
+      crow[k] = SW ? (unsigned)((size_t)sw_row(i) * rowbytes)
+                   : (unsigned)((min((int)blockIdx.x * 128 + i, a.Npad - 1) - (int)blockIdx.x * 128) * rowbytes);
+    }
+    // dword index of this lane in a plane: [32 groups][SB][2]
+    const int pidx = (SB == 4 ? wave : wave & 1) * 64 + lane;
+    const int pg = pidx / (2 * SB);
+    const size_t pbase = SW ? 0 : (size_t)blockIdx.x * 32 * a.B * 8;
+    const unsigned prow =
+        SW ? (unsigned)((size_t)(sw_row(4 * pg) >> 2) * a.B * 8)
+           : (unsigned)((min((int)blockIdx.x * 32 + pg, a.Npad / 4 - 1) - (int)blockIdx.x * 32) * a.B * 8);
+    const unsigned pq = (unsigned)(pidx % (2 * SB)) * 4, plast = (unsigned)a.B * 8 - 4;
+    auto dma_codes = [&](int gb, int slot, int k) {
+      dma_to_lds_s<16>(cbase, crow[k] + min(gb * W::CB + cq[k], clast),
+                       __builtin_amdgcn_readfirstlane(lbase + WOFF + (2 * wave + k) * 1024) + slot * W::BYTES);
+    };
+    auto dma_plane = [&](int gb, int slot, const uint16_t *plane, int which) {
+      dma_to_lds_s<4>(reinterpret_cast<const uint8_t *>(plane) + pbase, prow + min(gb * 8 + pq, plast),
+                      __builtin_amdgcn_readfirstlane(lbase + WOFF + W::CODES + which * W::PLANE +
+                                                     (SB == 4 ? wave : wave & 1) * 256) +
+                          slot * W::BYTES);
+    };
+    // Part ph (of SB) of a group's DMAs, so they spread over its blocks: NW
+    // instructions a part, so one wait count fits every step (Q4_0 and Q8_0
+    // repeat the scales in their last part).
+    constexpr int NW = SB == 4 ? 1 : 2;
+    auto dma_w = [&](int gb, int slot, int ph) {
+      if (ph == 0) {
+        dma_codes(gb, slot, 0);
+        if constexpr (SB == 1) dma_codes(gb, slot, 1);
+        if constexpr (SB == 2) dma_plane(gb, slot, a.dsc, 0);
+      } else if (ph == 1) {
+        dma_codes(gb, slot, 1);
+        if constexpr (SB == 2) dma_plane(gb, slot, a.dsc, 0);
+      } else if (ph == 2 || W::NSC == 1) {
+        dma_plane(gb, slot, a.dsc, 0);
+      } else {
+        dma_plane(gb, slot, a.msc, 1);
+      }
+    };
+    // this lane's read offsets in an activation stage and in a weight group
+    const uint8_t *rbase = &S[0];
+    int aoff[TT][2];
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r = m0 + 32 * t + lr;
+        aoff[t][j] = (r * 32 + (((2 * j + h) ^ a_swz(r)) * 8)) * 2;
+      }
+    const unsigned wswz = a_swz(lr) * 16;  // the same for the rows 32 and 64 further on
+    const unsigned wrow = WOFF + (wn * 64 + lr) * 64 + (TYPE == PBX_F16 ? 0 : 8 * h);
+    const unsigned prd = WOFF + W::CODES + ((wn * 16 + (lr >> 2)) * SB * 4 + (lr & 3)) * 2;
+
+    // A block's operands in registers: the activation fragments (hi and lo of
+    // each half block), the weight bytes as read, then as MFMA operands.
+    half8 Af[TT][4];                    // hi 0, hi 1, lo 0, lo 1
+    half8 Bf[2][2];
+    float d[2], mn[2];
+    auto read_a = [&](int slot, half8 (&A)[TT][4]) {
+      const uint8_t *sb = rbase + slot * STAGE;
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        A[t][0] = *reinterpret_cast<const half8 *>(sb + aoff[t][0]);
+        A[t][2] = *reinterpret_cast<const half8 *>(sb + PS + aoff[t][0]);
+        A[t][1] = *reinterpret_cast<const half8 *>(sb + aoff[t][1]);
+        A[t][3] = *reinterpret_cast<const half8 *>(sb + PS + aoff[t][1]);
+      }
+    };
+    // block ph of the weight group at byte offset wo of the ring
+    auto read_w = [&](unsigned wo, unsigned ph, uint4 (&raw)[2][2], float (&dd)[2], float (&mm)[2]) {
+      const uint8_t *sb = rbase + wo;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const uint8_t *wr = sb + wrow + 2048 * u;
+        if constexpr (TYPE == PBX_F16) {
+          raw[u][0] = *reinterpret_cast<const uint4 *>(wr + ((16 * h) ^ wswz));
+          raw[u][1] = *reinterpret_cast<const uint4 *>(wr + ((32 + 16 * h) ^ wswz));
+          dd[u] = 1.f;
+          mm[u] = 0.f;
+        } else {
+          const uint2 r0 = *reinterpret_cast<const uint2 *>(wr + ((ph * W::CB) ^ wswz));
+          const uint2 r1 = TYPE == PBX_Q8
+                               ? *reinterpret_cast<const uint2 *>(wr + ((ph * W::CB + 16) ^ wswz))
+                               : r0;
+          raw[u][0] = make_uint4(r0.x, r0.y, 0u, 0u);
+          raw[u][1] = make_uint4(r1.x, r1.y, 0u, 0u);
+          const uint8_t *pr = sb + prd + ph * 8 + SB * 64 * u;
+          dd[u] = f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(pr));
+          mm[u] = TYPE == PBX_Q41
+                      ? f16_bits_to_f32(*reinterpret_cast<const uint16_t *>(pr + W::PLANE))
+                      : 0.f;
+        }
+      }
+    };
+    auto unpack = [&](const uint4 (&raw)[2][2], half8 (&Bo)[2][2]) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          if constexpr (TYPE == PBX_F16)
+            Bo[u][j] = __builtin_bit_cast(half8, raw[u][j]);
+          else  // Q4: low nibbles for j = 0, high for j = 1
+            Bo[u][j] = codes_operand<TYPE>(make_uint2(raw[u][j].x, raw[u][j].y),
+                                           TYPE == PBX_Q8 ? 0 : 2 * j);
+        }
+    };
+
+    // The block loop is pipelined over registers: while block b multiplies,
+    // block b + 1's operands are read from LDS and its codes unpacked, and the
+    // scale FMAs of a pair of 32 x 32 products run under the next pair's
+    // MFMAs (pend: the products not yet scaled).
+    floatx16 pend[2] = {zero16, zero16};
+    float pd[2] = {0.f, 0.f};
+    auto scale_pending = [&](int t) {
+      if constexpr (TYPE != PBX_F16) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            acc[t][u][r] = fmaf(pend[u][r], pd[u], acc[t][u][r]);
+          }
+      }
+    };
+
+    // groups fetched ahead of the current block's; a group of one block takes
+    // the slot of the block just read, like the activations
+    constexpr int AHEAD = SB == 1 ? 3 : 2;
+    auto dma_group = [&](int g) {
+#pragma unroll
+      for (int p = 0; p < SB; ++p) dma_w(b0 + g * SB, g, p);
+    };
+    dma_group(0);
+    dma_x(b0, 0);
+    dma_x(min(b0 + 1, b1 - 1), 1);
+    dma_group(1);
+    dma_x(min(b0 + 2, b1 - 1), 2);
+    if constexpr (AHEAD == 3) dma_group(2);
+    wait_vm<4 * NA + (AHEAD - 1) * SB * NW>();
+    lds_barrier();
+    {
+      uint4 raw[2][2];
+      read_a(0, Af);
+      read_w(0, 0, raw, d, mn);
+      unpack(raw, Bf);
+    }
+    // weight ring: the group being read (offset and block of the next read)
+    // and the group being fetched (AHEAD groups after the current block's)
+    unsigned rd_ph = SB == 1 ? 0 : 1, rd_off = SB == 1 ? W::BYTES : 0;
+    int is_ph = 0, is_slot = AHEAD % 3;
+
+    for (int kb = b0; kb < b1; kb += 3) {
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        const int b = kb + s;
+        if (b >= b1) break;
+        // All but the last step's DMAs have arrived, block b + 1's operands
+        // among them (its activations were requested two steps ago), and
+        // every wave holds block b in registers: its slot is refilled with
+        // block b + 3.
+        wait_vm<2 * NA + NW>();
+        lds_barrier();
+        dma_x(min(b + 3, b1 - 1), s);
+        dma_w(b + AHEAD * SB - is_ph, is_slot, is_ph);
+        half8 An[TT][4], Bn[2][2];
+        uint4 raw[2][2];
+        float dn[2], mnn[2];
+        read_w(rd_off, rd_ph, raw, dn, mnn);
+        read_a(s == 2 ? 0 : s + 1, An);
+        if (++rd_ph == SB) {
+          rd_ph = 0;
+          rd_off = rd_off == 2 * W::BYTES ? 0 : rd_off + W::BYTES;
+        }
+        if (++is_ph == SB) {
+          is_ph = 0;
+          is_slot = is_slot == 2 ? 0 : is_slot + 1;
+        }
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          if constexpr (TYPE == PBX_F16) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+              for (int u = 0; u < 2; ++u)
+                acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Af[t][((q & 1) << 1) | (q >> 1)], Bf[u][q >> 1], acc[t][u], 0, 0, 0);
+          } else {
+            floatx16 blk[2] = {zero16, zero16}, xs = zero16;
+            if constexpr (TYPE == PBX_Q41) {
+              // the block sums of the activation rows: the product with all-ones weights
+              half8 ones;
+#pragma unroll
+              for (int e = 0; e < 8; ++e) ones[e] = (_Float16)1.f;
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                xs = __builtin_amdgcn_mfma_f32_32x32x16_f16(Af[t][((q & 1) << 1) | (q >> 1)], ones, xs, 0, 0, 0);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+              for (int u = 0; u < 2; ++u)
+                blk[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Af[t][((q & 1) << 1) | (q >> 1)], Bf[u][q >> 1], blk[u], 0, 0, 0);
+            scale_pending(t == 0 ? TT - 1 : t - 1);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              pend[u] = blk[u];
+              pd[u] = d[u];
+              if constexpr (TYPE == PBX_Q41) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[t][u][r] = fmaf(xs[r], mn[u], acc[t][u][r]);
+              }
+            }
+          }
+        }
+        unpack(raw, Bn);
+        // issue order of the step: an MFMA, an LDS read, six vector operations
+#pragma unroll
+        for (int i = 0; i < 8 * TT; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) Af[t][q] = An[t][q];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          Bf[u][0] = Bn[u][0];
+          Bf[u][1] = Bn[u][1];
+          d[u] = dn[u];
+          mn[u] = mnn[u];
+        }
+      }
+    }
+    scale_pending(TT - 1);
+    wait_vm<0>();
+  }
+
+  store_tiles<SW, TT>(a, acc, mblk + m0, n0, wn, lr, h);
+}
+
+// 64-row tiles: a ring of NS LDS stages, each [hi/lo][64 rows][4 chunks of 8
+// halves] of activations, the 128 weight rows' code bytes (or F16 weights) of
+// one block and their scales (and Q4_1 mins); wave tile 32 x 64.  The loop is
+// unrolled by NS so every LDS offset is an immediate.
+// Weight bytes of one row and block in the stage: Q4_0 / Q4_1 16 code bytes,
+// Q8_0 32, F16 64 (the fp16 weights); per-block scales (and Q4_1 mins) follow.
+template <int TYPE> struct DmaB {
+  static constexpr int CB = TYPE == PBX_F16 ? 64 : TYPE == PBX_Q8 ? 32 : 16;
+  static constexpr int CODES = 128 * CB;                  // bytes of a stage
+  static constexpr int NSC = TYPE == PBX_F16 ? 0 : TYPE == PBX_Q41 ? 2 : 1;  // 256-byte planes
+  static constexpr int WD = TYPE == PBX_Q8 || TYPE == PBX_F16 ? 2 : 1;      // weight DMAs a wave
+};
+
+template <int TYPE, bool SW = false>
+__device__ __forceinline__ void gemm_dma64(const GemmArgs &a) {
+  constexpr int MT = 64, NS = 3;
+  typedef DmaB<TYPE> W;
   constexpr int NA = MT / 64;                                     // activation chunks a wave and plane
   constexpr int TT = MT / 64;                                     // 32-row MFMA tiles a wave
   constexpr int PS = MT * 32 * 2;                                 // bytes of a stage's hi (or lo) plane
@@ -357,7 +738,6 @@ __device__ __forceinline__ void gemm_dma(const GemmArgs &a) {
   const int n0 = blockIdx.x * 128 + wn * 64;
   const int mblk = blockIdx.y * MT;
   const int m0 = wm * (MT / 2);
-  const int K = a.B * 32;
   const int per = (a.B + a.KS - 1) / a.KS;
   const int b0 = blockIdx.z * per;
   const int b1 = min(a.B, b0 + per);
@@ -377,10 +757,11 @@ __device__ __forceinline__ void gemm_dma(const GemmArgs &a) {
     for (int i = 0; i < NA; ++i) {
       const int c = (4 * i + wave) * 64 + lane;  // plane 0 chunk (same offsets in plane 1)
       const int r = c >> 2, q = (c & 3) ^ a_swz(r);
-      avoff[i] = (unsigned)((r * K + q * 8) * 2);
+      avoff[i] = (unsigned)((r * 32 + q * 8) * 2);
     }
-    const uint8_t *xhi = reinterpret_cast<const uint8_t *>(a.X16 + (size_t)mblk * K);
-    const uint8_t *xlo = reinterpret_cast<const uint8_t *>(a.X16lo + (size_t)mblk * K);
+    const size_t xstep = (size_t)a.Mpad * 64;  // bytes of a block
+    const uint8_t *xhi = reinterpret_cast<const uint8_t *>(a.X16) + (size_t)mblk * 64;
+    const uint8_t *xlo = reinterpret_cast<const uint8_t *>(a.X16lo) + (size_t)mblk * 64;
     // Weight DMAs of this wave (bases at the workgroup's first row, so the
     // per-lane offsets stay small).  Code DMA d moves 1 KB: rows
     // (1024 / CB) d + lane / (CB / 16), 16-byte chunk lane % (CB / 16), into
@@ -450,10 +831,10 @@ __device__ __forceinline__ void gemm_dma(const GemmArgs &a) {
     auto dma = [&](int b, int stage) {
       const unsigned so = stage * STAGE;
 #pragma unroll
-      for (int i = 0; i < NA; ++i) dma_to_lds_s<16>(xhi + b * 64, avoff[i], lds0 + so + 4096 * i);
+      for (int i = 0; i < NA; ++i) dma_to_lds_s<16>(xhi + b * xstep, avoff[i], lds0 + so + 4096 * i);
 #pragma unroll
       for (int i = 0; i < NA; ++i)
-        dma_to_lds_s<16>(xlo + b * 64, avoff[i], lds0 + so + PS + 4096 * i);
+        dma_to_lds_s<16>(xlo + b * xstep, avoff[i], lds0 + so + PS + 4096 * i);
 #pragma unroll
       for (int k = 0; k < W::WD; ++k) {
         if (wsz[k] == 16)
@@ -553,64 +934,29 @@ __device__ __forceinline__ void gemm_dma(const GemmArgs &a) {
     wait_vm<0>();
   }
 
-  if constexpr (SW) {
-    const int NO = a.N / 2, c = blockIdx.x * 64 + 32 * wn + lr;  // the lane's hidden column
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = mblk + m0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (m < a.M) {
-          const float iv = a.inv[m];
-          a.Y[(size_t)m * NO + c] = silu(acc[t][0][r] * iv) * (acc[t][1][r] * iv);
-        }
-      }
-    return;
-  }
-#pragma unroll
-  for (int t = 0; t < TT; ++t)
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int n = n0 + 32 * u + lr;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = mblk + m0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (m < a.M && n < a.N) {
-          const float v = acc[t][u][r] * a.inv[m];
-          if (a.KS == 1) {
-            float *y = a.Y + (size_t)m * a.N + n;
-            if (a.accumulate)
-              *y += v;
-            else
-              *y = v + (a.bias ? a.bias[n] : 0.f);
-          } else {
-            a.Y[((size_t)blockIdx.z * a.M + m) * a.N + n] = v;
-          }
-        }
-      }
-    }
+  store_tiles<SW, TT>(a, acc, mblk + m0, n0, wn, lr, h);
 }
 
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_big(GemmArgs a) { gemm_dma<PBX_Q4, 3>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_big(GemmArgs a) { gemm_dma<PBX_Q8, 3>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_big(GemmArgs a) { gemm_dma<PBX_Q41, 3>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_big(GemmArgs a) { gemm_dma<PBX_F16, 3>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_big(GemmArgs a) { gemm_dma<PBX_Q4>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_big(GemmArgs a) { gemm_dma<PBX_Q8>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_big(GemmArgs a) { gemm_dma<PBX_Q41>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_big(GemmArgs a) { gemm_dma<PBX_F16>(a); }
 // 64-row M tiles: twice the workgroups of the 128-row tile for the GEMMs
 // whose 128 x 128 grid leaves CUs idle (o, q|k|v and down at a 512-token
 // prompt), without a deeper K split
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_b64(GemmArgs a) { gemm_dma<PBX_Q4, 3, 64>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_b64(GemmArgs a) { gemm_dma<PBX_Q8, 3, 64>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_b64(GemmArgs a) { gemm_dma<PBX_Q41, 3, 64>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_b64(GemmArgs a) { gemm_dma<PBX_F16, 3, 64>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_b64(GemmArgs a) { gemm_dma64<PBX_Q4>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_b64(GemmArgs a) { gemm_dma64<PBX_Q8>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_b64(GemmArgs a) { gemm_dma64<PBX_Q41>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_b64(GemmArgs a) { gemm_dma64<PBX_F16>(a); }
 // gate|up with silu(gate) * up in the epilogue (no K split; Y is [M][N / 2])
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_big_sw(GemmArgs a) { gemm_dma<PBX_Q4, 3, 128, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_big_sw(GemmArgs a) { gemm_dma<PBX_Q8, 3, 128, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_big_sw(GemmArgs a) { gemm_dma<PBX_Q41, 3, 128, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_big_sw(GemmArgs a) { gemm_dma<PBX_F16, 3, 128, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_b64_sw(GemmArgs a) { gemm_dma<PBX_Q4, 3, 64, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_b64_sw(GemmArgs a) { gemm_dma<PBX_Q8, 3, 64, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_b64_sw(GemmArgs a) { gemm_dma<PBX_Q41, 3, 64, true>(a); }
-extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_b64_sw(GemmArgs a) { gemm_dma<PBX_F16, 3, 64, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_big_sw(GemmArgs a) { gemm_dma<PBX_Q4, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_big_sw(GemmArgs a) { gemm_dma<PBX_Q8, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_big_sw(GemmArgs a) { gemm_dma<PBX_Q41, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_big_sw(GemmArgs a) { gemm_dma<PBX_F16, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_b64_sw(GemmArgs a) { gemm_dma64<PBX_Q4, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_b64_sw(GemmArgs a) { gemm_dma64<PBX_Q8, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_b64_sw(GemmArgs a) { gemm_dma64<PBX_Q41, true>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_b64_sw(GemmArgs a) { gemm_dma64<PBX_F16, true>(a); }
 
 // Row scaling to fp16: one workgroup per (padded) row.  The scale is
 // 2^(15 - e) with 2^(e-1) <= max|x| < 2^e, so every scaled value is below
@@ -623,11 +969,17 @@ extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_b64_sw(GemmArgs a
 #define PREP_R 8
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 
+// Row m of X16 is 64 bytes of every block of Mpad rows ([K / 32][Mpad][32],
+// Mpad = the grid): its float4 k as half4v index, relative to the row's start
+__device__ __forceinline__ size_t prep_at(int k) {
+  return (size_t)(k >> 3) * gridDim.x * 8 + (k & 7);
+}
+
 __device__ __forceinline__ void prep_zero_row(_Float16 *dst, _Float16 *lo, float *inv, int K4) {
   const half4v z = {};
   for (int k = threadIdx.x; k < K4; k += 256) {
-    reinterpret_cast<half4v *>(dst)[k] = z;
-    reinterpret_cast<half4v *>(lo)[k] = z;
+    reinterpret_cast<half4v *>(dst)[prep_at(k)] = z;
+    reinterpret_cast<half4v *>(lo)[prep_at(k)] = z;
   }
   if (threadIdx.x == 0) *inv = 0.f;
 }
@@ -669,8 +1021,8 @@ __device__ __forceinline__ void prep_split_row(const float4 (&v)[PREP_R], int K4
       const half4v hv = {(_Float16)a0, (_Float16)a1, (_Float16)a2, (_Float16)a3};
       const half4v lv = {(_Float16)(a0 - (float)hv[0]), (_Float16)(a1 - (float)hv[1]),
                          (_Float16)(a2 - (float)hv[2]), (_Float16)(a3 - (float)hv[3])};
-      reinterpret_cast<half4v *>(dst)[k] = hv;
-      reinterpret_cast<half4v *>(lo)[k] = lv;
+      reinterpret_cast<half4v *>(dst)[prep_at(k)] = hv;
+      reinterpret_cast<half4v *>(lo)[prep_at(k)] = lv;
     }
   }
   if (tid == 0) *inv = mx > 0.f ? ldexpf(1.f, e - 15) : 1.f;
@@ -711,7 +1063,7 @@ extern "C" __global__ void __launch_bounds__(256)
 pbx_gemm_prep_x(const float *X, _Float16 *X16, _Float16 *X16lo, float *inv, int M, int K) {
   __shared__ float red[4];
   const int m = blockIdx.x, K4 = K / 4;  // K is a multiple of 32, at most 1024 * PREP_R
-  _Float16 *dst = X16 + (size_t)m * K, *lo = X16lo + (size_t)m * K;
+  _Float16 *dst = X16 + (size_t)m * 32, *lo = X16lo + (size_t)m * 32;
   if (m >= M) return prep_zero_row(dst, lo, inv + m, K4);
   if (K4 > 256 * PREP_R) {
     // longer rows: read twice
@@ -731,8 +1083,8 @@ pbx_gemm_prep_x(const float *X, _Float16 *X16, _Float16 *X16lo, float *inv, int 
       const half4v hv = {(_Float16)a0, (_Float16)a1, (_Float16)a2, (_Float16)a3};
       const half4v lv = {(_Float16)(a0 - (float)hv[0]), (_Float16)(a1 - (float)hv[1]),
                          (_Float16)(a2 - (float)hv[2]), (_Float16)(a3 - (float)hv[3])};
-      reinterpret_cast<half4v *>(dst)[k] = hv;
-      reinterpret_cast<half4v *>(lo)[k] = lv;
+      reinterpret_cast<half4v *>(dst)[prep_at(k)] = hv;
+      reinterpret_cast<half4v *>(lo)[prep_at(k)] = lv;
     }
     if (threadIdx.x == 0) inv[m] = mx > 0.f ? ldexpf(1.f, e - 15) : 1.f;
     return;
@@ -748,7 +1100,7 @@ pbx_gemm_prep_rms(const float *X, const float *normw, float eps, _Float16 *X16, 
                   float *inv, int M, int K) {
   __shared__ float red[4];
   const int m = blockIdx.x, K4 = K / 4;
-  _Float16 *dst = X16 + (size_t)m * K, *lo = X16lo + (size_t)m * K;
+  _Float16 *dst = X16 + (size_t)m * 32, *lo = X16lo + (size_t)m * 32;
   if (m >= M) return prep_zero_row(dst, lo, inv + m, K4);
   float4 v[PREP_R];
   load_row(X + (size_t)m * K, K4, v);
@@ -764,7 +1116,7 @@ pbx_gemm_reduce_rms(const float *part, int KS, float *X, const float *normw, flo
                     _Float16 *X16, _Float16 *X16lo, float *inv, int M, int K) {
   __shared__ float red[4];
   const int m = blockIdx.x, K4 = K / 4;
-  _Float16 *dst = X16 + (size_t)m * K, *lo = X16lo + (size_t)m * K;
+  _Float16 *dst = X16 + (size_t)m * 32, *lo = X16lo + (size_t)m * 32;
   if (m >= M) {
     if (normw) prep_zero_row(dst, lo, inv + m, K4);
     return;
@@ -807,7 +1159,7 @@ pbx_gemm_prep_swiglu(const float *GU, _Float16 *X16, _Float16 *X16lo, float *inv
                      int hidden) {
   __shared__ float red[4];
   const int m = blockIdx.x, K4 = hidden / 4;
-  _Float16 *dst = X16 + (size_t)m * hidden, *lo = X16lo + (size_t)m * hidden;
+  _Float16 *dst = X16 + (size_t)m * 32, *lo = X16lo + (size_t)m * 32;
   if (m >= M) return prep_zero_row(dst, lo, inv + m, K4);
   const float4 *g4 = reinterpret_cast<const float4 *>(GU + (size_t)m * 2 * hidden);
   const float4 *u4 = g4 + K4;

@@ -21,6 +21,7 @@ struct GemmArgsHost {  // GemmArgs in pbx_gemm.hip
   int M, N, Npad, B, KS;
   int accumulate;
   const void *msc;
+  int Mpad;
 };
 
 struct GemmF32ArgsHost {  // GemmF32Args in pbx_gemm.hip
@@ -166,14 +167,12 @@ int pbx_gemm_make_plan(pbx_ctx *c, const pbx_weight *w, int M, pbx_gemm_plan *p,
   int mtl = mtiles;
   if (big) {
     // 128 x 128 tiles where they give two workgroups a CU (the prefill's
-    // gate|up); otherwise 64-row M tiles (pbx_gemm_<type>_b64) with the K
-    // split to two workgroups a CU (PBX_GEMM_M64 = workgroups a CU, 0: the
-    // 128-row tiles at about one a CU).  512-token prefill: 4.34 against
-    // 4.48 ms (q|k|v 37.3 -> 32.2 us, o 25 -> 22.5 us; down unchanged);
-    // three or four a CU: 4.48 and 4.67 ms.  With 128-row tiles a deeper
-    // split costs more in partial traffic and per-workgroup start-up than
-    // the extra occupancy returns (measured against 0.5, 0.75, 1.5, 2 and 3
-    // per CU).
+    // gate|up): 16384 x 2048 at 2000 rows 312 us against 337 in 64-row tiles
+    // (half the outputs for the same codes unpacked).  Otherwise
+    // 64-row M tiles (pbx_gemm_<type>_b64) with the K split to two workgroups
+    // a CU (PBX_GEMM_M64 = workgroups a CU, 0: the 128-row tiles at about one
+    // a CU): 8192 x 2048 at 512 rows 57.7 against 63.1 us in 128-row tiles at
+    // one a CU, 3072 x 2048 at 2000 80 against 86.
     const int wgs = nwg * mtiles;
     const char *e = getenv("PBX_GEMM_M64");
     const int per_cu = e ? atoi(e) : 2;
@@ -215,7 +214,7 @@ int pbx_gemm_run(pbx_ctx *c, const pbx_weight *w, const pbx_gemm_plan &p, const 
   hipFunction_t fg = pbx_kernel_by_name(c, p.name);
   if (!fg) return pbx_fail(c, PBX_ELOAD, "pbx_gemm: kernel %s missing", p.name.c_str());
   GemmArgsHost g{w->qs, w->d, x16, x16lo, inv, p.KS == 1 ? dBias : nullptr, out,
-                 p.M, (int)w->N, (int)w->Npad, (int)w->B, p.KS, p.KS == 1 ? accumulate : 0, w->m};
+                 p.M, (int)w->N, (int)w->Npad, (int)w->B, p.KS, p.KS == 1 ? accumulate : 0, w->m, p.Mpad};
   void *args[] = {&g};
   return pbx_launch_fn(c, fg, p.name.c_str(), dim3(p.nwg, p.mtiles, p.KS), dim3(256), args, stream);
 }

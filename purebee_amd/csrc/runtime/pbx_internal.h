@@ -171,7 +171,7 @@ int pbx_linear_enqueue(pbx_ctx *c, const pbx_weight *w, const float *dX, int64_t
 #define PBX_SCRATCH_BYTES ((size_t)PBX_NOALLOC_WORKSPACE_BYTES)
 int pbx_scratch_lookup(pbx_ctx *c);
 // The fp16 MFMA GEMM in two parts, for callers that prepare the fp16
-// activation pair (X16, X16lo, inv: [Mpad][K]) themselves: the kernel, grid
+// activation pair (X16, X16lo: [K / 32][Mpad][32], inv: [Mpad]) themselves: the kernel, grid
 // and K split for M rows of weight w, and the launch, which writes Y (KS == 1,
 // += if accumulate) or the KS partials [KS][M][N].
 struct pbx_gemm_plan {
