@@ -94,12 +94,27 @@ __device__ __forceinline__ void load_codes(const GemmArgs &a, int n, int b, int 
   }
 }
 
+// Eight byte codes c (< 256; bytes 0-3 of x, then of y) as fp16 c + 1024 - bias.
+// One v_perm_b32 builds the fp16 pair [0x64 | byte e, 0x64 | byte e+1] =
+// 1024 + c (exact: fp16 spacing is 1 on [1024, 2048)) from the code bytes and
+// the constant 0x64 bytes, and one packed-fp16 subtract removes the bias.
+__device__ __forceinline__ half8 bytes_operand(unsigned x, unsigned y, _Float16 bias) {
+  auto pair = [&](unsigned v, unsigned sel) -> half2v {
+    // selector bytes 0..3 pick v's bytes, 4 picks a 0x64 byte of the constant
+    const unsigned h = __builtin_amdgcn_perm(0x64646464u, v, sel);
+    return __builtin_bit_cast(half2v, h) - half2v{bias, bias};
+  };
+  const half2v p0 = pair(x, 0x04010400u), p1 = pair(x, 0x04030402u);
+  const half2v p2 = pair(y, 0x04010400u), p3 = pair(y, 0x04030402u);
+  half8 v;
+  v[0] = p0[0]; v[1] = p0[1]; v[2] = p1[0]; v[3] = p1[1];
+  v[4] = p2[0]; v[5] = p2[1]; v[6] = p3[0]; v[7] = p3[1];
+  return v;
+}
+
 // The 8 weights as an fp16 MFMA operand: the integer codes q - 8 (Q4_0,
 // low nibbles for g < 2, high for g >= 2), q (Q4_1, same nibbles) or q
-// (Q8_0), or the F16 weights themselves.  One v_perm_b32 builds the fp16 pair
-// [0x64 | byte e, 0x64 | byte e+1] = 1024 + c (exact: fp16 spacing is 1 on
-// [1024, 2048)) from the code bytes and the constant 0x64 bytes, and one
-// packed-fp16 subtract removes 1024 + bias.  Nibbles are isolated in their
+// (Q8_0), or the F16 weights themselves.  Nibbles are isolated in their
 // bytes first; Q8_0 int8 codes are made unsigned (q + 128).
 template <int TYPE>
 __device__ __forceinline__ half8 codes_operand(typename RawT<TYPE>::type w, int g) {
@@ -118,17 +133,7 @@ __device__ __forceinline__ half8 codes_operand(typename RawT<TYPE>::type w, int 
       y ^= 0x80808080u;
       bias = (_Float16)1152.f;  // 1024 + 128
     }
-    auto pair = [&](unsigned v, unsigned sel) -> half2v {
-      // selector bytes 0..3 pick v's bytes, 4 picks a 0x64 byte of the constant
-      const unsigned h = __builtin_amdgcn_perm(0x64646464u, v, sel);
-      return __builtin_bit_cast(half2v, h) - half2v{bias, bias};
-    };
-    const half2v p0 = pair(x, 0x04010400u), p1 = pair(x, 0x04030402u);
-    const half2v p2 = pair(y, 0x04010400u), p3 = pair(y, 0x04030402u);
-    half8 v;
-    v[0] = p0[0]; v[1] = p0[1]; v[2] = p1[0]; v[3] = p1[1];
-    v[4] = p2[0]; v[5] = p2[1]; v[6] = p3[0]; v[7] = p3[1];
-    return v;
+    return bytes_operand(x, y, bias);
   }
 }
 
@@ -269,6 +274,287 @@ GEMM_KERNEL(pbx_gemm_f16_m1_n2, PBX_F16, 1, 2)
 GEMM_KERNEL(pbx_gemm_f16_m1_n4, PBX_F16, 1, 4)
 GEMM_KERNEL(pbx_gemm_f16_m2_n2, PBX_F16, 2, 2)
 
+
+// ---------------------------------------------------------------------------
+// Few rows in one launch (pbx_gemm_rows_<type>_m<MT>_n<NT>): Y = X . W^T
+// straight from the fp32 activations, no preparation, no partials.  A
+// workgroup owns 16 * MT rows of X and 16 * NT rows of W; its waves take the
+// chunks of 8 blocks (256 columns) in turn and meet in LDS.  A wave scales
+// each activation row of its chunk by a power of two (largest magnitude just
+// below 2^15; undone exactly when the chunk is added) and splits it into the
+// fp16 pair (hi, lo) of the kernels above, so a value keeps at least the bits
+// that the whole-row scale gives it.
+// Lane group g = l / 16 takes k = 8g + e of a block, in Q4_0 / Q4_1 the
+// elements 4g + e and 16 + 4g + e of the dword 4g (both nibbles, no byte read
+// twice).  Q6_K scales its codes by 16s: lanes g < 2 hold the first 16, so a
+// block is two products whose other half is zeroed.
+// Q4_0 8192 x 2048 at 16 rows: 12 us a call against 16.9 with preparation,
+// split GEMM and reduction as three launches (floor 2 us: one launch and the
+// latency of a chunk's loads are the rest); Q6_K 128256 x 2048 at 5 rows 72 us
+// against 350 with one GEMV pass a row (3.0 TB/s, the code unpacking beside the
+// loads bounds it).
+// ---------------------------------------------------------------------------
+#define ROWS_WV 8  // waves of a workgroup at most
+
+struct GemmRowsArgs {
+  const uint8_t *qs;
+  const uint16_t *dsc;
+  const uint16_t *msc;
+  const float *X;     // [M][K]
+  const float *bias;  // [N] or null
+  float *Y;           // [M][N]
+  int M, N, Npad, B;
+  int accumulate;
+};
+
+// One chunk's weight bytes of one weight row in a lane.
+template <int TYPE> struct RowsW { typedef unsigned code_t; static constexpr int NC = 8; };
+template <> struct RowsW<PBX_Q8> { typedef uint2 code_t; static constexpr int NC = 8; };
+template <> struct RowsW<PBX_F16> { typedef uint4 code_t; static constexpr int NC = 8; };
+// [half][ql of groups 0 / 2, ql of groups 1 / 3, qh]
+template <> struct RowsW<PBX_Q6K> { typedef uint2 code_t; static constexpr int NC = 6; };
+
+__device__ __forceinline__ float max4(float4 t) {
+  return fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w)));
+}
+
+// LOOP: at most 8 chunks, one a wave, whose activations stay in registers as
+// the fp16 pair while the workgroup walks every gridDim.x-th tile of W, the
+// next tile's bytes in flight.
+template <int TYPE, int MT, int NT, bool LOOP>
+__device__ __forceinline__ void gemm_rows(const GemmRowsArgs &a) {
+  typedef RowsW<TYPE> W;
+  constexpr bool NIB = TYPE == PBX_Q4 || TYPE == PBX_Q41;
+  constexpr bool Q6 = TYPE == PBX_Q6K;
+  __shared__ float red[LOOP ? 2 : 1][ROWS_WV][MT * NT][256];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const int li = lane & 15, g = lane >> 4;
+  const int m0 = blockIdx.y * (16 * MT);
+  const int B = a.B, K = B * 32, chunks = (B + 7) / 8;
+  const int tiles = (a.N + 16 * NT - 1) / (16 * NT);
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  // the lane's two float4 of a block
+  const int x0 = NIB ? 4 * g : 8 * g, x1 = NIB ? 16 + 4 * g : 8 * g + 4;
+
+  // A chunk's weight bytes of NT weight rows, as loaded.
+  struct Raw {
+    typename W::code_t w[NT][W::NC];
+    unsigned d[NT][Q6 ? 1 : 8], m[NT][TYPE == PBX_Q41 ? 8 : 1];
+    uint2 sc[NT][Q6 ? 2 : 1];
+  };
+  auto load_w = [&](int tile, int c, Raw &q) {
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      const int n = min(tile * (16 * NT) + 16 * u + li, a.Npad - 1);
+      if constexpr (Q6) {
+        const uint8_t *blk = a.qs + ((size_t)n * (B >> 3) + c) * PBX_Q6K_BYTES;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          q.w[u][3 * hf] = *reinterpret_cast<const uint2 *>(blk + 64 * hf + 8 * g);
+          q.w[u][3 * hf + 1] = *reinterpret_cast<const uint2 *>(blk + 64 * hf + 32 + 8 * g);
+          q.w[u][3 * hf + 2] = *reinterpret_cast<const uint2 *>(blk + 128 + 32 * hf + 8 * g);
+          q.sc[u][hf] = *reinterpret_cast<const uint2 *>(blk + 192 + 8 * hf);
+        }
+        q.d[u][0] = a.dsc[dsc_index(n, c, B >> 3)];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int b = min(c * 8 + j, B - 1);
+          const size_t blk = (size_t)n * B + b;
+          q.w[u][j] = *reinterpret_cast<const typename W::code_t *>(
+              NIB ? a.qs + blk * 16 + 4 * g
+                  : TYPE == PBX_Q8 ? a.qs + blk * 32 + 8 * g : a.qs + (blk * 32 + 8 * g) * 2);
+          if constexpr (TYPE != PBX_F16) q.d[u][j] = a.dsc[dsc_index(n, b, B)];
+          if constexpr (TYPE == PBX_Q41) q.m[u][j] = a.msc[dsc_index(n, b, B)];
+        }
+      }
+    }
+  };
+  // A chunk's activations: the fp16 pair of every block (blocks past the last
+  // are copies of it, not multiplied) and the power of two that undoes the
+  // row's scale.
+  float4 xv[MT][8][2];
+  half8 Ah[MT][8], Al[MT][8];
+  float inv[MT];
+  auto load_x = [&](int c) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const float *row = a.X + (size_t)min(m0 + 16 * t + li, a.M - 1) * K;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float *p = row + min(c * 8 + j, B - 1) * 32;
+        xv[t][j][0] = *reinterpret_cast<const float4 *>(p + x0);
+        xv[t][j][1] = *reinterpret_cast<const float4 *>(p + x1);
+      }
+    }
+  };
+  auto split_x = [&]() {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      float mx = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fmaxf(max4(xv[t][j][0]), max4(xv[t][j][1])));
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      int e = 0;
+      if (mx > 0.f && mx < INFINITY) frexpf(mx, &e);
+      e = max(e, -110);  // both powers of two stay normal numbers
+      const float scale = ldexpf(1.f, 15 - e);
+      inv[t] = ldexpf(1.f, e - 15);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v[8] = {xv[t][j][0].x, xv[t][j][0].y, xv[t][j][0].z, xv[t][j][0].w,
+                            xv[t][j][1].x, xv[t][j][1].y, xv[t][j][1].z, xv[t][j][1].w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float s = v[i] * scale;
+          Ah[t][j][i] = (_Float16)s;
+          Al[t][j][i] = (_Float16)(s - (float)Ah[t][j][i]);
+        }
+      }
+    }
+  };
+  floatx4 total[MT][NT];
+  // total += the chunk's products, the row scales undone (output row 4g + r
+  // has lane 4g + r's)
+  auto multiply = [&](int c, const Raw &q) {
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < NT; ++u) acc[t][u] = zero;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (c * 8 + j < B) {
+        floatx4 xs[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          xs[t] = TYPE == PBX_Q41 ? block_sums(Ah[t][j], Al[t][j]) : zero;
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+          if constexpr (Q6) {
+            const int hf = j >> 2, grp = j & 3;
+            const uint2 l = q.w[u][3 * hf + (grp & 1)], hq = q.w[u][3 * hf + 2];
+            auto code = [&](unsigned lo, unsigned hi) -> unsigned {
+              const unsigned hb = grp == 0 ? hi << 4 : grp == 1 ? hi << 2 : grp == 2 ? hi : hi >> 2;
+              return ((lo >> (grp >> 1) * 4) & 0x0F0F0F0Fu) | (hb & 0x30303030u);
+            };
+            const uint4 w = __builtin_bit_cast(
+                uint4, bytes_operand(code(l.x, hq.x), code(l.y, hq.y), (_Float16)1056.f));
+            const unsigned k0 = g < 2 ? ~0u : 0u, k1 = ~k0;
+            const half8 W0 = __builtin_bit_cast(half8, make_uint4(w.x & k0, w.y & k0, w.z & k0, w.w & k0));
+            const half8 W1 = __builtin_bit_cast(half8, make_uint4(w.x & k1, w.y & k1, w.z & k1, w.w & k1));
+            const unsigned sb = (grp < 2 ? q.sc[u][hf].x : q.sc[u][hf].y) >> (grp & 1) * 16;
+            const float d = f16_bits_to_f32(q.d[u][0]);
+            const float d0 = d * (float)(int8_t)(sb & 255u), d1 = d * (float)(int8_t)((sb >> 8) & 255u);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+              floatx4 p0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[t][j], W0, zero, 0, 0, 0);
+              floatx4 p1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[t][j], W1, zero, 0, 0, 0);
+              p0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[t][j], W0, p0, 0, 0, 0);
+              p1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[t][j], W1, p1, 0, 0, 0);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[t][u][r] = fmaf(p1[r], d1, fmaf(p0[r], d0, acc[t][u][r]));
+            }
+          } else {
+            half8 Wop;
+            float d = 1.f, mn = 0.f;
+            if constexpr (NIB)
+              Wop = bytes_operand(q.w[u][j] & 0x0F0F0F0Fu, (q.w[u][j] >> 4) & 0x0F0F0F0Fu,
+                                  TYPE == PBX_Q4 ? (_Float16)1032.f : (_Float16)1024.f);
+            else
+              Wop = codes_operand<TYPE>(q.w[u][j], 0);
+            if constexpr (TYPE != PBX_F16) d = f16_bits_to_f32(q.d[u][j]);
+            if constexpr (TYPE == PBX_Q41) mn = f16_bits_to_f32(q.m[u][j]);
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+              block_mma<TYPE>(acc[t][u], Ah[t][j], Al[t][j], Wop, d, mn, xs[t]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float iv = __shfl(inv[t], 4 * g + r);
+#pragma unroll
+        for (int u = 0; u < NT; ++u) total[t][u][r] = fmaf(acc[t][u][r], iv, total[t][u][r]);
+      }
+  };
+  auto clear = [&]() {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < NT; ++u) total[t][u] = zero;
+  };
+  // the waves' sums, added in wave order
+  auto finish = [&](int tile, float (&rd)[ROWS_WV][MT * NT][256]) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rd[wave][t * NT + u][(4 * g + r) * 16 + li] = total[t][u][r];
+    lds_barrier();
+    for (int i = threadIdx.x; i < MT * NT * 256; i += blockDim.x) {
+      const int nc = i % (16 * NT), mr = i / (16 * NT);  // column and row of the tile
+      const int m = m0 + mr, n = tile * (16 * NT) + nc;
+      if (m >= a.M || n >= a.N) continue;
+      const int tu = (mr >> 4) * NT + (nc >> 4), at = (mr & 15) * 16 + (nc & 15);
+      float v = rd[0][tu][at];
+      for (int k = 1; k < nw; ++k) v += rd[k][tu][at];
+      float *y = a.Y + (size_t)m * a.N + n;
+      *y = a.accumulate ? *y + v : v + (a.bias ? a.bias[n] : 0.f);
+    }
+  };
+
+  if constexpr (LOOP) {
+    Raw q;
+    load_x(wave);
+    load_w(blockIdx.x, wave, q);
+    split_x();
+    int buf = 0;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+      Raw next;
+      load_w(min(tile + (int)gridDim.x, tiles - 1), wave, next);
+      clear();
+      multiply(wave, q);
+      finish(tile, red[buf]);  // two buffers: the one read last is refilled after the next barrier
+      buf ^= 1;
+      q = next;
+    }
+  } else {
+    clear();
+    for (int c = wave; c < chunks; c += nw) {
+      Raw q;
+      load_x(c);
+      load_w(blockIdx.x, c, q);
+      split_x();
+      multiply(c, q);
+    }
+    finish(blockIdx.x, red[0]);
+  }
+}
+
+#define ROWS_KERNEL(TAG, TYPE, MT, NT, SUF, LOOP)                                    \
+  extern "C" __global__ void __launch_bounds__(64 * ROWS_WV)                         \
+      pbx_gemm_rows_##TAG##_m##MT##_n##NT##SUF(GemmRowsArgs a) {                     \
+    gemm_rows<TYPE, MT, NT, LOOP>(a);                                                \
+  }
+#define ROWS_KERNELS(TAG, TYPE)          \
+  ROWS_KERNEL(TAG, TYPE, 1, 1, , false)  \
+  ROWS_KERNEL(TAG, TYPE, 1, 2, , false)  \
+  ROWS_KERNEL(TAG, TYPE, 1, 4, , false)  \
+  ROWS_KERNEL(TAG, TYPE, 2, 2, , false)  \
+  ROWS_KERNEL(TAG, TYPE, 1, 2, l, true)  \
+  ROWS_KERNEL(TAG, TYPE, 2, 1, l, true)
+ROWS_KERNELS(q4, PBX_Q4)
+ROWS_KERNELS(q8, PBX_Q8)
+ROWS_KERNELS(q41, PBX_Q41)
+ROWS_KERNELS(f16, PBX_F16)
+ROWS_KERNELS(q6k, PBX_Q6K)
 
 // ---------------------------------------------------------------------------
 // Large-M kernel (M > 32): 32x32x16 MFMAs with every operand moved to LDS
@@ -990,10 +1276,6 @@ __device__ __forceinline__ float block_sum256(float v, float *red) {
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-__device__ __forceinline__ float max4(float4 t) {
-  return fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w)));
 }
 
 // Scale and split the row v (element 4 (tid + 256 i) + c of float4 i) into

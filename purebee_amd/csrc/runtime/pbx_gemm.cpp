@@ -33,6 +33,17 @@ struct GemmF32ArgsHost {  // GemmF32Args in pbx_gemm.hip
   int accumulate;
 };
 
+struct GemmRowsArgsHost {  // GemmRowsArgs in pbx_gemm.hip
+  const void *qs;
+  const void *dsc;
+  const void *msc;
+  const float *X;
+  const float *bias;
+  float *Y;
+  int M, N, Npad, B;
+  int accumulate;
+};
+
 const char *gemm_tag(int type) {
   switch (type) {
     case PBX_TYPE_Q4_0: return "q4";
@@ -134,6 +145,53 @@ int launch_f32(pbx_ctx *c, const pbx_weight *w, const float *dX, int M, const fl
   return launch_reduce(c, part, dBias, dY, M, N, KS, accumulate, stream);
 }
 
+// Few activation rows, one launch: 16 * MT rows of X and 16 * NT rows of W a
+// workgroup.
+int launch_rows(pbx_ctx *c, const pbx_weight *w, const float *dX, int M, const float *dBias,
+                float *dY, int accumulate, hipStream_t stream) {
+  const int N = (int)w->N, B = (int)w->B, chunks = (B + 7) / 8;
+  // Every workgroup loads and splits its activations, so the widest tile wins
+  // that still gives three quarters of the CUs a workgroup: 8192 x 2048 at 16
+  // rows 12.0 us with NT = 2 (256 workgroups) against 15.0 with NT = 1; 2048 x
+  // 8192 at 32 rows 28 us in 16 x 16 tiles (256) against 37 and 43 in 16 x 32
+  // and 32 x 16; 3072 x 2048 at 32 rows 12.0 in 16 x 32 (192) against 14.7.
+  auto wgs = [&](int mt, int nt) {
+    return (int64_t)((N + 16 * nt - 1) / (16 * nt)) * ((M + 16 * mt - 1) / (16 * mt));
+  };
+  const int64_t enough = c->cu_count * 3 / 4;
+  int MT = 1, NT = 1;
+  if (M > 16 && wgs(2, 2) >= enough) MT = NT = 2;
+  else if (M <= 16 && wgs(1, 4) >= enough) NT = 4;
+  else if (wgs(1, 2) >= enough) NT = 2;
+  // More than one round of workgroups: those of one a CU walk the tiles with
+  // the activations in registers (K <= 2048).  16384 x 2048 Q8_0 at 20 rows
+  // 21.6 us against 28.6; 128256 x 2048 Q6_K at 5 rows 72 against 98.
+  const bool loop = chunks <= 8 && NT > 1 && wgs(MT, NT) >= 2 * c->cu_count;
+  if (loop) NT = MT == 1 ? 2 : 1;
+  const std::string name = std::string("pbx_gemm_rows_") +
+                           (w->type == PBX_TYPE_Q6_K ? "q6k" : gemm_tag(w->type)) + "_m" +
+                           std::to_string(MT) + "_n" + std::to_string(NT) + (loop ? "l" : "");
+  hipFunction_t f = pbx_kernel_by_name(c, name);
+  if (!f) return pbx_fail(c, PBX_ELOAD, "pbx_gemm: kernel %s missing", name.c_str());
+  const int tiles = (N + 16 * NT - 1) / (16 * NT), mtiles = (M + 16 * MT - 1) / (16 * MT);
+  GemmRowsArgsHost g{w->qs, w->d, w->m, dX, dBias, dY, M, N, (int)w->Npad, B, accumulate};
+  void *args[] = {&g};
+  return pbx_launch_fn(c, f, name.c_str(),
+                       dim3(loop ? std::min(tiles, std::max(1, c->cu_count / mtiles)) : tiles, mtiles),
+                       dim3(64 * std::min(8, chunks)), args, stream);
+}
+
+// Workspace of the prepared GEMM: the fp16 pair, the row scales and the
+// split-K partials.
+struct GemmSpace {
+  size_t x16, inv, part;
+  size_t total() const { return 2 * x16 + inv + part; }
+};
+GemmSpace gemm_space(const pbx_gemm_plan &p, int N, int K) {
+  return {((size_t)p.Mpad * K * 2 + 255) / 256 * 256, ((size_t)p.Mpad * 4 + 255) / 256 * 256,
+          p.KS > 1 ? (size_t)p.KS * p.M * N * 4 : 0};
+}
+
 }  // namespace
 
 int pbx_gemm_make_plan(pbx_ctx *c, const pbx_weight *w, int M, pbx_gemm_plan *p, bool swiglu) {
@@ -222,26 +280,32 @@ int pbx_gemm_run(pbx_ctx *c, const pbx_weight *w, const pbx_gemm_plan &p, const 
 int pbx_gemm_launch(pbx_ctx *c, const pbx_weight *w, const float *dX, int64_t M64,
                     const float *dBias, float *dY, int accumulate, hipStream_t stream,
                     const pbx_workspace *wsp) {
-  if (!gemm_tag(w->type))
+  if (!gemm_tag(w->type) && w->type != PBX_TYPE_Q6_K)
     return pbx_fail(c, PBX_ENOTSUP, "pbx_gemm: weight type %d has no MFMA path", w->type);
   if (M64 > 65535) return pbx_fail(c, PBX_ENOTSUP, "pbx_gemm: M=%lld too large", (long long)M64);
   if (w->type == PBX_TYPE_F32)
     return launch_f32(c, w, dX, (int)M64, dBias, dY, accumulate, stream, wsp);
+  if (w->type == PBX_TYPE_Q6_K) {
+    if (w->B > 512)
+      return pbx_fail(c, PBX_ENOTSUP, "pbx_linear: K=%lld exceeds the Q6_K limit of 16384",
+                      (long long)w->K);
+    return launch_rows(c, w, dX, (int)M64, dBias, dY, accumulate, stream);
+  }
+  if (M64 <= 32 && !wsp) return launch_rows(c, w, dX, (int)M64, dBias, dY, accumulate, stream);
   const int M = (int)M64, N = (int)w->N, K = (int)w->B * 32;
   pbx_gemm_plan p;
   int rc = pbx_gemm_make_plan(c, w, M, &p);
   if (rc) return rc;
-  // fp16 activations and their fp16 rounding residuals
-  const size_t x16_bytes = ((size_t)p.Mpad * K * 2 + 255) / 256 * 256;
-  const size_t lo_bytes = x16_bytes;
-  const size_t inv_bytes = ((size_t)p.Mpad * 4 + 255) / 256 * 256;
-  const size_t part_bytes = p.KS > 1 ? (size_t)p.KS * M * N * 4 : 0;
+  const GemmSpace sp = gemm_space(p, N, K);
   char *ws = nullptr;
-  if ((rc = workspace(c, wsp, x16_bytes + lo_bytes + inv_bytes + part_bytes, &ws))) return rc;
+  if ((rc = workspace(c, wsp, sp.total(), &ws))) return rc;
+  // (a caller's workspace limits the shapes the same way with either kernel)
+  if (M <= 32) return launch_rows(c, w, dX, M, dBias, dY, accumulate, stream);
+  // fp16 activations and their fp16 rounding residuals
   void *x16 = ws;
-  void *x16lo = ws + x16_bytes;
-  float *inv = (float *)(ws + x16_bytes + lo_bytes);
-  float *part = (float *)(ws + x16_bytes + lo_bytes + inv_bytes);
+  void *x16lo = ws + sp.x16;
+  float *inv = (float *)(ws + 2 * sp.x16);
+  float *part = (float *)(ws + 2 * sp.x16 + sp.inv);
   hipFunction_t fprep = pbx_kernel_by_name(c, "pbx_gemm_prep_x");
   if (!fprep) return pbx_fail(c, PBX_ELOAD, "pbx_gemm: kernel pbx_gemm_prep_x missing");
   {

@@ -541,9 +541,7 @@ int pbx_linear_enqueue(pbx_ctx *c, const pbx_weight *w, const float *dX, int64_t
     return pbx_launch(c, PBX_K_GEMV_Q8REF, dim3((unsigned)((N + 63) / 64), gy), dim3(512),
                       args, stream);
   }
-  // Q6_K rows stay on the GEMV kernels for every M (one grid row per
-  // activation row); the MFMA GEMM covers the other types.
-  if (M >= PBX_GEMM_MIN_M && w->type != PBX_TYPE_Q6_K)
+  if (M >= PBX_GEMM_MIN_M)
     return pbx_gemm_enqueue(c, w, dX, M, dBias, dY, stream, ws);
   int B = (int)w->B;
   // Integer-limb kernels (gemv_int) for Q4_0 / Q8_0 with K = 2048..8192 (not

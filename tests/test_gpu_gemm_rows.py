@@ -1,0 +1,100 @@
+"""The one-launch GEMM for few activation rows (and every M of Q6_K): tile
+edges in M and N, chunks of 8 blocks with a remainder, fewer chunks than
+waves and more, the form that walks the tiles (tall N, K <= 2048).  Every row
+within 1e-5 relative L2 of the oracle: activations keep 2^-22 of their row's
+largest magnitude in a chunk, sums are fp32."""
+import numpy as np
+import pytest
+
+import oracle
+import purebee_amd as pb
+from tests.conftest import rel_l2
+from tests.test_gpu_gemv import synth_matrix, weight_bytes
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [pb.TYPE_Q4_0, pb.TYPE_Q8_0, pb.TYPE_Q4_1, pb.TYPE_F16, pb.TYPE_Q6_K]
+
+
+def raw_weights(t, seed, N, K):
+    W = synth_matrix(seed, N, K)
+    return oracle.quantize_q6_k(W) if t == pb.TYPE_Q6_K else weight_bytes(t, W)
+
+
+def activations(M, K, seed):
+    X = pb.synth_normal(seed, M * K).reshape(M, K)
+    X[1] *= 1e-30
+    X[2] *= 1e30
+    X[3, : K // 2] *= 1e-4  # chunks of very different magnitude
+    return X
+
+
+def error(y, ref, x):
+    """Relative L2 error; a few outputs can cancel to far less than the sums
+    that they are made of (one output of row 0.02 * |x| typical size came out
+    at 8e-4), whose rounding stays in proportion to |w| |x|, so the norm is
+    taken as at least that of outputs without cancellation."""
+    typical = 0.02 * np.linalg.norm(x.astype(np.float64)) * np.sqrt(len(ref))
+    return np.linalg.norm(y.astype(np.float64) - ref) / max(np.linalg.norm(ref), typical)
+
+
+def check(ctx, t, M, N, K, rows):
+    print(f"[case] rows gemm type={t} M={M} N={N} K={K}", flush=True)
+    raw = raw_weights(t, 3 * N + K + M, N, K)
+    X = activations(M, K, M + N)
+    bias = pb.synth_normal(3, N)
+    w = ctx.upload(t, N, K, raw)
+    Y, Yb = ctx.linear(w, X), ctx.linear(w, X, bias)
+    w.free()
+    for m in rows:
+        ref = oracle.matvec(t, X[m], raw, N, K)
+        assert error(Y[m], ref, X[m]) <= 1e-5
+        if m not in (1, 2):  # the bias swamps or vanishes beside those rows
+            assert error(Yb[m], ref + bias, X[m]) <= 1e-5
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("M", [4, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(1, 256), (17, 512), (130, 2304), (3080, 256), (6200, 2560)])
+def test_rows_tiles(ctx, t, M, N, K):
+    check(ctx, t, M, N, K, [0, 1, 2, 3, M - 1])
+
+
+@pytest.mark.parametrize("t", TYPES[:4])
+@pytest.mark.parametrize("K", [32, 224, 288, 2080])
+def test_rows_partial_chunks(ctx, t, K):
+    check(ctx, t, 9, 50, K, [0, 1, 2, 3, 8])
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("M,N,K", [(5, 33000, 256), (20, 16500, 512)])
+def test_rows_tile_loop(ctx, t, M, N, K):
+    check(ctx, t, M, N, K, [0, 1, 2, 3, M - 1])
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 100, 256), (70, 300, 2304), (200, 2500, 512), (700, 48, 1024)])
+def test_q6_k_many_rows(ctx, M, N, K):
+    check(ctx, pb.TYPE_Q6_K, M, N, K, [0, 1, 2, 3, 31, 32, M - 1])
+
+
+@pytest.mark.parametrize("t", TYPES)
+def test_rows_non_finite_stays_in_its_row(ctx, t):
+    M, N, K = 6, 40, 2304
+    raw = raw_weights(t, 5, N, K)
+    X = pb.synth_normal(8, M * K).reshape(M, K)
+    X[2, 7] = np.inf
+    X[4, 300] = np.nan
+    w = ctx.upload(t, N, K, raw)
+    Y = ctx.linear(w, X)
+    w.free()
+    assert not np.isfinite(Y[2]).any() and np.isnan(Y[4]).all()
+    for m in (0, 1, 3, 5):
+        assert rel_l2(Y[m], oracle.matvec(t, X[m], raw, N, K)) <= 1e-5
+
+
+def test_q6_k_k_limit_is_refused(ctx):
+    N, K = 2, 16640
+    w = ctx.upload(pb.TYPE_Q6_K, N, K, raw_weights(pb.TYPE_Q6_K, 1, N, K))
+    with pytest.raises(pb.PbxError):
+        ctx.linear(w, np.zeros((4, K), np.float32))
+    w.free()
