@@ -11,9 +11,8 @@
 //   A: lane l holds A[l%16][8*(l/16) + e], e = 0..7
 //   B: lane l holds B[8*(l/16) + e][l%16]
 //   D: lane l holds D[4*(l/16) + r][l%16], r = 0..3
-// For Q4_0 lane group g = l/16 takes k = 8g..8g+7 of the block: low nibbles
-// of bytes 0..7 (g=0), of bytes 8..15 (g=1), high nibbles of bytes 0..7
-// (g=2) and of bytes 8..15 (g=3), the element order of gguf.js:259-286.
+// (gemm_rows, up to 32 rows and Q6_K; the larger forms below take two
+// v_mfma_f32_32x32x16_f16 a block).  Elements in the order of gguf.js:259-286.
 //
 // Precision: weights enter the MFMA as their integer codes (q - 8 for Q4_0,
 // q for Q8_0, q for Q4_1) or, for F16, as themselves, which fp16 holds
@@ -54,45 +53,10 @@ struct GemmArgs {
 
 namespace {
 
-// Two byte-sized codes c0, c1 (< 256, in bits 0-7 and 8-15 of v) as fp16
-// 1024 + c (exact: fp16 spacing is 1 on [1024, 2048)), minus `bias`.
-__device__ __forceinline__ half2v codes_to_half2(unsigned v, _Float16 bias) {
-  const unsigned p = (v & 0xFFu) | ((v & 0xFF00u) << 8) | 0x64006400u;
-  return __builtin_bit_cast(half2v, p) - half2v{bias, bias};
-}
-
 // Per-lane operand bytes of one block: 8 codes (8 bytes) for the quantised
 // types, 8 fp16 weights (16 bytes) for F16.
 template <int TYPE> struct RawT { typedef uint2 type; };
 template <> struct RawT<PBX_F16> { typedef uint4 type; };
-
-// Raw bytes of lane group g's 8 weights of row n, block b, and the block's
-// scale (and Q4_1 min) bits; zero for padding rows.
-template <int TYPE>
-__device__ __forceinline__ void load_codes(const GemmArgs &a, int n, int b, int g,
-                                           typename RawT<TYPE>::type *raw, unsigned *dbits,
-                                           unsigned *mbits) {
-  if (n >= a.Npad) {
-    *raw = {};
-    *dbits = 0u;
-    *mbits = 0u;
-    return;
-  }
-  if constexpr (TYPE == PBX_F16) {
-    *raw = *reinterpret_cast<const uint4 *>(a.qs + (((size_t)n * a.B + b) * 32 + 8 * g) * 2);
-    *dbits = 0x3C00u;  // 1.0
-    *mbits = 0u;
-    return;
-  } else {
-    const size_t di = dsc_index(n, b, a.B);
-    *dbits = a.dsc[di];
-    *mbits = TYPE == PBX_Q41 ? a.msc[di] : 0u;
-    if constexpr (TYPE == PBX_Q4 || TYPE == PBX_Q41)
-      *raw = *reinterpret_cast<const uint2 *>(a.qs + ((size_t)n * a.B + b) * 16 + (g & 1) * 8);
-    else
-      *raw = *reinterpret_cast<const uint2 *>(a.qs + ((size_t)n * a.B + b) * 32 + g * 8);
-  }
-}
 
 // Eight byte codes c (< 256; bytes 0-3 of x, then of y) as fp16 c + 1024 - bias.
 // One v_perm_b32 builds the fp16 pair [0x64 | byte e, 0x64 | byte e+1] =
@@ -168,112 +132,7 @@ __device__ __forceinline__ floatx4 block_sums(half8 Ah, half8 Al) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, ones, s, 0, 0, 0);
 }
 
-// Workgroup = 4 waves side by side along n.  Wave tile: 16*MT rows of X by
-// 16*NT rows of W; blockIdx.z splits the K blocks.  The block loop runs in
-// steps of U blocks whose loads are all issued before the first MFMA, so a
-// wave keeps U blocks of weights in flight.
-template <int TYPE, int MT, int NT, int U>
-__device__ __forceinline__ void gemm_tile(const GemmArgs &a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int li = lane & 15, g = lane >> 4;
-  const int n0 = (blockIdx.x * 4 + wave) * (16 * NT);
-  const int m0 = blockIdx.y * (16 * MT);
-  const int per = (a.B + a.KS - 1) / a.KS;
-  const int b0 = blockIdx.z * per;
-  const int b1 = min(a.B, b0 + per);
-  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-
-  floatx4 acc[MT][NT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int u = 0; u < NT; ++u) acc[t][u] = zero;
-
-  for (int b = b0; b < b1; b += U) {
-    typename RawT<TYPE>::type raw[U][NT];
-    unsigned dbits[U][NT], mbits[U][NT];
-    half8 A[U][MT], Alo[U][MT];
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      const int bb = b + j;
-      if (bb < b1) {
-#pragma unroll
-        for (int u = 0; u < NT; ++u)
-          load_codes<TYPE>(a, n0 + 16 * u + li, bb, g, &raw[j][u], &dbits[j][u], &mbits[j][u]);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          const size_t off = ((size_t)bb * a.Mpad + m0 + 16 * t + li) * 32 + 8 * g;
-          A[j][t] = *reinterpret_cast<const half8 *>(a.X16 + off);
-          Alo[j][t] = *reinterpret_cast<const half8 *>(a.X16lo + off);
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      if (b + j < b1) {
-        floatx4 xs[MT];
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-          xs[t] = TYPE == PBX_Q41 ? block_sums(A[j][t], Alo[j][t]) : zero;
-#pragma unroll
-        for (int u = 0; u < NT; ++u) {
-          const half8 W = codes_operand<TYPE>(raw[j][u], g);
-          const float d = f16_bits_to_f32(dbits[j][u]);
-          const float mn = f16_bits_to_f32(mbits[j][u]);
-#pragma unroll
-          for (int t = 0; t < MT; ++t) block_mma<TYPE>(acc[t][u], A[j][t], Alo[j][t], W, d, mn, xs[t]);
-        }
-      }
-    }
-  }
-
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int u = 0; u < NT; ++u) {
-      const int n = n0 + 16 * u + li;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + 16 * t + 4 * g + r;
-        if (m < a.M && n < a.N) {
-          const float v = acc[t][u][r] * a.inv[m];
-          if (a.KS == 1) {
-            float *y = a.Y + (size_t)m * a.N + n;
-            if (a.accumulate)
-              *y += v;
-            else
-              *y = v + (a.bias ? a.bias[n] : 0.f);
-          } else {
-            a.Y[((size_t)blockIdx.z * a.M + m) * a.N + n] = v;
-          }
-        }
-      }
-    }
-}
-
 }  // namespace
-
-#define GEMM_KERNEL(NAME, TYPE, MT, NT)                                            \
-  extern "C" __global__ void __launch_bounds__(256) NAME(GemmArgs a) {             \
-    gemm_tile<TYPE, MT, NT, (MT == 1 ? 8 : 2)>(a);                                  \
-  }
-GEMM_KERNEL(pbx_gemm_q4_m1_n1, PBX_Q4, 1, 1)
-GEMM_KERNEL(pbx_gemm_q4_m1_n2, PBX_Q4, 1, 2)
-GEMM_KERNEL(pbx_gemm_q4_m1_n4, PBX_Q4, 1, 4)
-GEMM_KERNEL(pbx_gemm_q4_m2_n2, PBX_Q4, 2, 2)
-GEMM_KERNEL(pbx_gemm_q8_m1_n1, PBX_Q8, 1, 1)
-GEMM_KERNEL(pbx_gemm_q8_m1_n2, PBX_Q8, 1, 2)
-GEMM_KERNEL(pbx_gemm_q8_m1_n4, PBX_Q8, 1, 4)
-GEMM_KERNEL(pbx_gemm_q8_m2_n2, PBX_Q8, 2, 2)
-GEMM_KERNEL(pbx_gemm_q41_m1_n1, PBX_Q41, 1, 1)
-GEMM_KERNEL(pbx_gemm_q41_m1_n2, PBX_Q41, 1, 2)
-GEMM_KERNEL(pbx_gemm_q41_m1_n4, PBX_Q41, 1, 4)
-GEMM_KERNEL(pbx_gemm_q41_m2_n2, PBX_Q41, 2, 2)
-GEMM_KERNEL(pbx_gemm_f16_m1_n1, PBX_F16, 1, 1)
-GEMM_KERNEL(pbx_gemm_f16_m1_n2, PBX_F16, 1, 2)
-GEMM_KERNEL(pbx_gemm_f16_m1_n4, PBX_F16, 1, 4)
-GEMM_KERNEL(pbx_gemm_f16_m2_n2, PBX_F16, 2, 2)
-
 
 // ---------------------------------------------------------------------------
 // Few rows in one launch (pbx_gemm_rows_<type>_m<MT>_n<NT>): Y = X . W^T

@@ -199,70 +199,43 @@ int pbx_gemm_make_plan(pbx_ctx *c, const pbx_weight *w, int M, pbx_gemm_plan *p,
     return pbx_fail(c, PBX_ENOTSUP, "pbx_gemm: weight type %d has no fp16 MFMA path", w->type);
   if (M <= 0 || M > 65535) return pbx_fail(c, PBX_ENOTSUP, "pbx_gemm: M=%d out of range", M);
   const int N = (int)w->N, B = (int)w->B;
-  // M > 32: the LDS-tiled 128 x 128 kernel; otherwise one wave per 16*MT
-  // rows x 16*NT weight rows.
-  const bool big = M > 32;
-  const int MT = big ? 8 : M <= 16 ? 1 : 2;
-  const int Mpad = (M + 16 * MT - 1) / (16 * MT) * (16 * MT);
-  const int mtiles = Mpad / (16 * MT);
-  const int want_wg = 2 * c->cu_count;
-  int NT, nwg;
-  if (big) {
-    NT = 8;
-    nwg = (N + 127) / 128;
-  } else {
-    // Largest n tile that still gives two workgroups per CU.
-    if (MT == 1)
-      NT = ((N + 255) / 256) * mtiles >= want_wg ? 4 : ((N + 127) / 128) * mtiles >= want_wg ? 2 : 1;
-    else
-      NT = 2;
-    nwg = (N + 64 * NT - 1) / (64 * NT);
-  }
-  // Split K so the grid has about one workgroup (big) or eight waves
-  // (small) per CU.
+  const int Mpad = (M + 127) / 128 * 128, mtiles = Mpad / 128, nwg = (N + 127) / 128;
   int KS = 1;
   int mt_rows = 128;
   int mtl = mtiles;
-  if (big) {
-    // 128 x 128 tiles where they give two workgroups a CU (the prefill's
-    // gate|up): 16384 x 2048 at 2000 rows 312 us against 337 in 64-row tiles
-    // (half the outputs for the same codes unpacked).  Otherwise
-    // 64-row M tiles (pbx_gemm_<type>_b64) with the K split to two workgroups
-    // a CU (PBX_GEMM_M64 = workgroups a CU, 0: the 128-row tiles at about one
-    // a CU): 8192 x 2048 at 512 rows 57.7 against 63.1 us in 128-row tiles at
-    // one a CU, 3072 x 2048 at 2000 80 against 86.
-    const int wgs = nwg * mtiles;
-    const char *e = getenv("PBX_GEMM_M64");
-    const int per_cu = e ? atoi(e) : 2;
-    if (per_cu > 0 && wgs < per_cu * c->cu_count) {
-      mt_rows = 64;
-      mtl = Mpad / 64;
-      const int w64 = nwg * mtl;
-      if (w64 < per_cu * c->cu_count)
-        KS = std::min({B, 8, (per_cu * c->cu_count + w64 - 1) / w64});
-    } else if (wgs < c->cu_count) {
-      KS = std::min({B, 8, (c->cu_count + wgs - 1) / wgs});
-    }
-  } else {
-    const int waves = nwg * mtiles * 4;
-    if (waves < 8 * c->cu_count) KS = std::min({B, 8, (8 * c->cu_count + waves - 1) / waves});
+  // 128 x 128 tiles where they give two workgroups a CU (the prefill's
+  // gate|up): 16384 x 2048 at 2000 rows 312 us against 337 in 64-row tiles
+  // (half the outputs for the same codes unpacked).  Otherwise
+  // 64-row M tiles (pbx_gemm_<type>_b64) with the K split to two workgroups
+  // a CU (PBX_GEMM_M64 = workgroups a CU, 0: the 128-row tiles at about one
+  // a CU): 8192 x 2048 at 512 rows 57.7 against 63.1 us in 128-row tiles at
+  // one a CU, 3072 x 2048 at 2000 80 against 86.
+  const int wgs = nwg * mtiles;
+  const char *e = getenv("PBX_GEMM_M64");
+  const int per_cu = e ? atoi(e) : 2;
+  if (per_cu > 0 && wgs < per_cu * c->cu_count) {
+    mt_rows = 64;
+    mtl = Mpad / 64;
+    const int w64 = nwg * mtl;
+    if (w64 < per_cu * c->cu_count)
+      KS = std::min({B, 8, (per_cu * c->cu_count + w64 - 1) / w64});
+  } else if (wgs < c->cu_count) {
+    KS = std::min({B, 8, (c->cu_count + wgs - 1) / wgs});
   }
   p->M = M;
   p->Mpad = Mpad;
   p->mtiles = mtl;
   p->nwg = nwg;
   p->KS = KS;
-  // gate|up with silu(gate) * up in the epilogue (M > 32 kernels, no K
-  // split, 64 hidden columns a workgroup, 32-bit weight offsets);
+  // gate|up with silu(gate) * up in the epilogue (no K split, 64
+  // hidden columns a workgroup, 32-bit weight offsets);
   // PBX_GEMM_SWIGLU=0 keeps gate and up side by side
   const char *sw_env = getenv("PBX_GEMM_SWIGLU");
-  p->swiglu = swiglu && big && KS == 1 && N % 128 == 0 &&
+  p->swiglu = swiglu && KS == 1 && N % 128 == 0 &&
               (double)N * pbx_type_row_bytes(w->type, w->K) < 4294967296.0 &&
               !(sw_env && sw_env[0] == '0');
   p->name = std::string("pbx_gemm_") + gemm_tag(w->type) +
-            (big ? std::string(mt_rows == 64 ? "_b64" : "_big")
-                 : "_m" + std::to_string(MT) + "_n" + std::to_string(NT)) +
-            (p->swiglu ? "_sw" : "");
+            (mt_rows == 64 ? "_b64" : "_big") + (p->swiglu ? "_sw" : "");
   return PBX_OK;
 }
 
@@ -291,16 +264,20 @@ int pbx_gemm_launch(pbx_ctx *c, const pbx_weight *w, const float *dX, int64_t M6
                       (long long)w->K);
     return launch_rows(c, w, dX, (int)M64, dBias, dY, accumulate, stream);
   }
-  if (M64 <= 32 && !wsp) return launch_rows(c, w, dX, (int)M64, dBias, dY, accumulate, stream);
   const int M = (int)M64, N = (int)w->N, K = (int)w->B * 32;
+  if (M <= PBX_GEMM_ROWS_M) {
+    // (no workspace needed; a caller's limits K as it does for more rows)
+    char *unused = nullptr;
+    const size_t pair = (size_t)(M <= 16 ? 16 : 32) * K * 4;
+    int rc = wsp ? workspace(c, wsp, pair, &unused) : PBX_OK;
+    return rc ? rc : launch_rows(c, w, dX, M, dBias, dY, accumulate, stream);
+  }
   pbx_gemm_plan p;
   int rc = pbx_gemm_make_plan(c, w, M, &p);
   if (rc) return rc;
   const GemmSpace sp = gemm_space(p, N, K);
   char *ws = nullptr;
   if ((rc = workspace(c, wsp, sp.total(), &ws))) return rc;
-  // (a caller's workspace limits the shapes the same way with either kernel)
-  if (M <= 32) return launch_rows(c, w, dX, M, dBias, dY, accumulate, stream);
   // fp16 activations and their fp16 rounding residuals
   void *x16 = ws;
   void *x16lo = ws + sp.x16;

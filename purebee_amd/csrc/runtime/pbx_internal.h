@@ -54,6 +54,9 @@ enum {
 
 // Row count from which quantized linears take the MFMA GEMM path.
 #define PBX_GEMM_MIN_M 4
+// Up to here the GEMM is one launch that reads the fp32 rows (launch_rows in
+// pbx_gemm.cpp); above, the prepared LDS-DMA GEMM.
+#define PBX_GEMM_ROWS_M 32
 
 #define PBX_MAX_MODULES 8
 
