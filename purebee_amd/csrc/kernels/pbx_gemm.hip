@@ -1318,19 +1318,47 @@ pbx_gemm_prep_swiglu(const float *GU, _Float16 *X16, _Float16 *X16lo, float *inv
   prep_split_row(v, K4, dst, lo, inv + m, red);
 }
 
-// Sum of the split-K partials (+ bias, or accumulated into Y).
+// Sum of the KS <= 8 split-K partials (+ bias, or accumulated into Y), in split
+// order; four outputs a thread.  Bound by the partials' bytes and their
+// latency: every partial is requested before the sum, 16 bytes each where rows
+// and pointers allow it (one float after the other took a call of 2048 x 8192
+// Q8_0 at 100 rows, 8 partials, 31.0 us against 30.0; 2048 x 2048 F32 at 512
+// rows, 4 partials, 44.8 against 44.0).
 extern "C" __global__ void __launch_bounds__(256)
 pbx_gemm_reduce(const float *part, const float *bias, float *Y, int M, int N, int KS,
                 int accumulate) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const int64_t MN = (int64_t)M * N;
   if (i >= MN) return;
-  float s = 0.f;
-  for (int k = 0; k < KS; ++k) s += part[k * MN + i];
-  if (accumulate)
-    Y[i] += s;
-  else
-    Y[i] = s + (bias ? bias[i % N] : 0.f);
+  if (N % 4 == 0 && (((uintptr_t)Y | (uintptr_t)bias | (uintptr_t)part) & 15) == 0) {
+    float4 pp[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      pp[k] = k < KS ? *reinterpret_cast<const float4 *>(part + k * MN + i)
+                     : make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 add = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (accumulate)
+      add = *reinterpret_cast<const float4 *>(Y + i);
+    else if (bias)
+      add = *reinterpret_cast<const float4 *>(bias + i % N);
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k < KS) {
+        s.x += pp[k].x; s.y += pp[k].y; s.z += pp[k].z; s.w += pp[k].w;
+      }
+    *reinterpret_cast<float4 *>(Y + i) =
+        make_float4(s.x + add.x, s.y + add.y, s.z + add.z, s.w + add.w);
+    return;
+  }
+  for (int64_t j = i; j < min(i + 4, MN); ++j) {
+    float s = 0.f;
+    for (int k = 0; k < KS; ++k) s += part[k * MN + j];
+    if (accumulate)
+      Y[j] += s;
+    else
+      Y[j] = s + (bias ? bias[j % N] : 0.f);
+  }
 }
 
 // ---------------------------------------------------------------------------

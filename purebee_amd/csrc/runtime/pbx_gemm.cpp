@@ -83,7 +83,7 @@ int launch_reduce(pbx_ctx *c, float *part, const float *dBias, float *dY, int M,
   int m = M, n = N, ks = KS, acc = accumulate;
   void *args[] = {&part, (void *)&dBias, &dY, &m, &n, &ks, &acc};
   const int64_t MN = (int64_t)M * N;
-  return pbx_launch_fn(c, fred, "pbx_gemm_reduce", dim3((unsigned)((MN + 255) / 256)), dim3(256),
+  return pbx_launch_fn(c, fred, "pbx_gemm_reduce", dim3((unsigned)((MN + 1023) / 1024)), dim3(256),
                        args, stream);
 }
 

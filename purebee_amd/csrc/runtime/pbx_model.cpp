@@ -1809,7 +1809,7 @@ static int fused_reduce(pbx_model *m, const pbx_gemm_plan &p, int N, float *Y, b
   int M = p.M, n = N, ks = p.KS, acc = accumulate ? 1 : 0;
   const int64_t total = (int64_t)M * N;
   void *args[] = {(void *)&part, (void *)&bias, &Y, &M, &n, &ks, &acc};
-  return launch_k(m, "pbx_gemm_reduce", dim3((unsigned)((total + 255) / 256)), dim3(256), args);
+  return launch_k(m, "pbx_gemm_reduce", dim3((unsigned)((total + 1023) / 1024)), dim3(256), args);
 }
 
 // x += the partials of the GEMM of plan p if it was split (p null: nothing to
