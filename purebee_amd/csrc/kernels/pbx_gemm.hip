@@ -58,6 +58,11 @@ namespace {
 template <int TYPE> struct RawT { typedef uint2 type; };
 template <> struct RawT<PBX_F16> { typedef uint4 type; };
 
+// Smallest row exponent e that the scales 2^(15 - e) and 2^(e - 15) are made
+// of: both stay normal numbers (unclamped, a row whose largest magnitude is
+// below 2^-113 was scaled by infinity, its zeros to NaN).
+#define ROW_EXP_MIN (-110)
+
 // Eight byte codes c (< 256; bytes 0-3 of x, then of y) as fp16 c + 1024 - bias.
 // One v_perm_b32 builds the fp16 pair [0x64 | byte e, 0x64 | byte e+1] =
 // 1024 + c (exact: fp16 spacing is 1 on [1024, 2048)) from the code bytes and
@@ -258,7 +263,7 @@ __device__ __forceinline__ void gemm_rows(const GemmRowsArgs &a) {
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       int e = 0;
       if (mx > 0.f && mx < INFINITY) frexpf(mx, &e);
-      e = max(e, -110);  // both powers of two stay normal numbers
+      e = max(e, ROW_EXP_MIN);
       const float scale = ldexpf(1.f, 15 - e);
       inv[t] = ldexpf(1.f, e - 15);
 #pragma unroll
@@ -1152,6 +1157,7 @@ __device__ __forceinline__ void prep_split_row(const float4 (&v)[PREP_R], int K4
   mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   int e = 0;
   if (mx > 0.f && mx < INFINITY) frexpf(mx, &e);
+  e = max(e, ROW_EXP_MIN);
   const float scale = mx > 0.f ? ldexpf(1.f, 15 - e) : 1.f;
 #pragma unroll
   for (int i = 0; i < PREP_R; ++i) {
@@ -1217,6 +1223,7 @@ pbx_gemm_prep_x(const float *X, _Float16 *X16, _Float16 *X16lo, float *inv, int 
     mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     int e = 0;
     if (mx > 0.f && mx < INFINITY) frexpf(mx, &e);
+    e = max(e, ROW_EXP_MIN);
     const float scale = mx > 0.f ? ldexpf(1.f, 15 - e) : 1.f;
     for (int k = threadIdx.x; k < K4; k += 256) {
       const float4 t = src[k];
@@ -1713,6 +1720,7 @@ __device__ __forceinline__ void skinny_q4(const SkinnyArgs &a) {
     const float vmax = x * r;  // the row's largest magnitude after normalisation
     int e = 0;
     if (vmax > 0.f && vmax < INFINITY) frexpf(vmax, &e);
+    e = max(e, ROW_EXP_MIN);
     rs_norm[m] = r;
     rs_scale[m] = vmax > 0.f ? ldexpf(1.f, 15 - e) : 1.f;
     rs_inv[m] = vmax > 0.f ? ldexpf(1.f, e - 15) : 1.f;

@@ -98,3 +98,27 @@ def test_q6_k_k_limit_is_refused(ctx):
     with pytest.raises(pb.PbxError):
         ctx.linear(w, np.zeros((4, K), np.float32))
     w.free()
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("M,K", [(6, 512), (40, 512), (130, 512), (40, 8448)])
+def test_tiny_rows_stay_finite(ctx, t, M, K):
+    """Rows whose largest magnitude lies below 2^-113, zeros among them: the
+    power of two that scales a row stays finite.  N(0, 1) times 1e-36 with
+    weights of 0.02: outputs around 1e-36, normal numbers; an activation keeps
+    2^-22 of itself (its fp16 pair at the clamped scale still holds 20 bits of
+    the row's largest magnitude), so 1e-5 as for the other rows.  K = 8448 is
+    the preparation of rows too long for the registers."""
+    N = 40
+    print(f"[case] tiny rows type={t} M={M} N={N} K={K}", flush=True)
+    raw = raw_weights(t, M + K, N, K)
+    X = pb.synth_normal(M, M * K).reshape(M, K)
+    X[1] *= 1e-36
+    X[1, 5::3] = 0.0
+    X[2] = 0.0
+    w = ctx.upload(t, N, K, raw)
+    Y = ctx.linear(w, X)
+    w.free()
+    assert np.isfinite(Y).all() and not Y[2].any()
+    for m in (0, 1, M - 1):
+        assert error(Y[m], oracle.matvec(t, X[m], raw, N, K), X[m]) <= 1e-5
