@@ -690,8 +690,10 @@ __device__ __forceinline__ void head_chunk_c(const float *kb, const float *vb, i
 
 // The same while the newest position nc - 1 is still being written: its
 // cache row is requested like the others, and its k and v (kn, vn: the
-// lane's dims) replace the loaded ones.  `ready` runs between the requests
-// and the arithmetic (the fused kernel waits there for q, kn and vn).
+// lane's dims) replace the loaded ones, in the rows past it too (clamped to
+// it: what the cache held there may not be finite, and a weight of 0 would
+// not keep it out of the sums).  `ready` runs between the requests and the
+// arithmetic (the fused kernel waits there for q, kn and vn).
 template <int J, class Ready>
 __device__ __forceinline__ void head_chunk_n(const float *kb, const float *vb, int kvdim, int dcol,
                                              int s0, int pl, int nc, Ready &&ready,
@@ -707,7 +709,7 @@ __device__ __forceinline__ void head_chunk_n(const float *kb, const float *vb, i
   ready();
 #pragma unroll
   for (int j = 0; j < J; ++j)
-    if (32 * (s0 + j) + pl == nc - 1) {
+    if (32 * (s0 + j) + pl >= nc - 1) {
       k[j] = kn;
       v[j] = vn;
     }
@@ -809,7 +811,7 @@ __device__ __forceinline__ void split_chunk(const float *kb, const float *vb, in
   ready();
 #pragma unroll
   for (int j = 0; j < J; ++j)
-    if (32 * (s0 + stride * j) + pl == nc - 1) {
+    if (32 * (s0 + stride * j) + pl >= nc - 1) {
       k[j] = kn;
       v[j] = vn;
     }

@@ -362,6 +362,47 @@ def test_non_finite_activation_propagates(ctx):
         ref.close()
 
 
+@pytest.mark.parametrize("path", ["joined", "split", "small"])
+def test_overwritten_non_finite_position(ctx, default_paths, path):
+    """A position that held a poisoned token (an embedding block of infinite
+    scale: its K and V are not finite) is decoded again with another token,
+    without a rollback: the logits are those of a model that never saw the
+    poisoned one, bit for bit.  The kernels that attend to the position while
+    its row is being written must take nothing from the row that was there,
+    also not for the slots past the end that are clamped to it."""
+    print(f"[case] poisoned position overwritten, {path}", flush=True)
+    monkeypatch = default_paths
+    from purebee_amd.native import T_TOKEN_EMBD
+    if path == "split":
+        monkeypatch.setenv("PBX_ATTN_SPLIT", "1")
+    if path == "small":
+        cfg, bb = tiny(TYPE_Q8_0, TYPE_Q8_0, n_layers=2), 34
+    else:
+        cfg, bb = tiny(TYPE_Q4_0, TYPE_Q4_0, dim=2048, hidden_dim=8192, n_layers=2, n_heads=32,
+                       n_kv_heads=8, vocab_size=512, max_seq=64), 18
+    bad = 7
+    emb = np.array(synth.make_tensor(synth.tensor_specs(cfg)[0], 141, 0), np.uint8, copy=True)
+    at = bad * (cfg["dim"] // 32) * bb
+    emb[at: at + 2] = np.frombuffer(np.uint16(0x7C00).tobytes(), np.uint8)
+    keep = np.arange(cfg["vocab_size"]) != bad  # tied head: the poisoned row's own logit
+    out = []
+    for poison in (False, True):
+        model = synth.build(ctx, cfg, 141)
+        model.set_tensor(T_TOKEN_EMBD, -1, emb)
+        for p in range(40):  # positions 2 and 36: a first slot and a second one
+            if poison and p in (2, 36):
+                assert not np.isfinite(model.forward([bad], p)[0]).any()
+            lg = model.forward([11 + p], p)[0]
+            if p in (2, 3, 36, 39):
+                out.append(lg[keep])
+        kern = {k for _, k, _, _ in model.profile(11, 40, 1)}
+        assert any(k.startswith("pbx_small_step" if path == "small" else "pbx_qkvr_attn_o_")
+                   for k in kern), kern
+        model.free()
+    for a, b in zip(out[:4], out[4:]):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
 def test_handoff_wait_timeout_is_reported(ctx, default_paths):
     """The bounded wait of the joined q|k|v + attention launch: when the
     cells it waits for never carry its tag (forced from the host by the test
