@@ -307,6 +307,13 @@ int pbx_model_op_name(const pbx_model *m, int i, char *buf, size_t cap);
  * PBX_ETIMEOUT.  layer < 0 restores the normal launch.  Returns
  * PBX_ENOTSUP when the model's step has no such launch. */
 int pbx_model_test_handoff(pbx_model *m, int layer, int skew, int spin);
+/* Test hook, no reference counterpart: in the joined launches that split a
+ * long context over workgroups, every workgroup expects its peers' states
+ * under tags `skew` epochs ahead (none ever arrive) and polls for them
+ * `spin` times (0: the kernel's default) before it computes them itself.
+ * Results stay the same, bit for bit.  skew 0 restores the normal launch.
+ * Returns PBX_ENOTSUP when the model's step has no such launch. */
+int pbx_model_test_peers(pbx_model *m, int skew, int spin);
 /* Measurement: the GEMV kernels of one role ("qkv", "o", "gate_up", "down",
  * "lm_head") launched back to back over every layer's weights, `reps`
  * passes between two HIP events on the model's stream; returns the mean

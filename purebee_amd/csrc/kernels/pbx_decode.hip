@@ -295,9 +295,12 @@ struct AttnArgs {
   unsigned long long *ocells;
   // pbx_qkvr_attn_o_*: contexts of more than split_at positions (0: none)
   // are split over the workgroups of a KV group, whose partial states travel
-  // as cells [n_heads][parts][PBX_PS_CELLS]
+  // as cells [n_heads][parts][PBX_PS_CELLS]; the tag offset that only a test
+  // sets (no peer's cell then ever matches) and the poll limit of a peer's
+  // state (0: PBX_PEER_SPIN)
   unsigned long long *pcells;
   int split_at;
+  int pskew, pspin;
 };
 
 // One workgroup per query head (llama.js:258-301 / llama-streaming.js:543-573):
@@ -781,8 +784,13 @@ __device__ __forceinline__ float poll_cell(const unsigned long long *cp, unsigne
 // and V leave the XCD's L2 once instead of 16 times.  A workgroup's state of
 // a head (weighted V sum, its maximum and sum) is published as cells tagged
 // like the q|k|v rows, and every workgroup then merges the 16 states of its
-// own head and goes on to its o rows.  All the workgroups must be resident
-// at once (the host checks the grid against the CUs); the waits are bounded.
+// own head and goes on to its o rows.
+// No workgroup depends on a peer: beside other launches (another stream's) a
+// group need not be resident as a whole, so a state that has not arrived
+// after PBX_PEER_SPIN polls is computed here (split_absent), with the peer's
+// own operations in their order, hence bit for bit the same.  (That code, though
+// hardly ever run, costs every launch 0.2 us: 317 -> 320 us a token at KV 128,
+// 413 -> 416 at 3500.)
 // Bound by the K/V transfer and by the hand-off's ~2 us: Llama-1B decode at KV
 // 3500 888 -> 403 us a token, 2000: 543 -> 371, 1000: 406 -> 361.  The hand-off
 // costs more than it saves on short contexts (700: 374 unsplit against 363, 512:
@@ -790,6 +798,7 @@ __device__ __forceinline__ float poll_cell(const unsigned long long *cp, unsigne
 #define PBX_PS_HEADS 4
 #define PBX_PS_CELLS 66  // 64 dims, maximum, sum
 #define PBX_PS_SLOTS 8   // slots in flight
+#define PBX_PEER_SPIN 128  // polls of a peer's state, some 100 us
 
 // J slots p + 16 j0 .. of the workgroup, folded into the four heads' states.
 template <int J, class Ready>
@@ -846,17 +855,68 @@ __device__ __forceinline__ void split_chunk(const float *kb, const float *vb, in
   }
 }
 
-// Leaves the states of query head h in st_m / st_l / st_acc (wave w holds the
-// merged states w and w + 8 of the head's `parts` <= 16 states).
+// LDS of a split context.
+struct SplitLds {
+  float rows[PBX_PS_HEADS + 2][PBX_HA_MAX_HD];  // q of the heads, new k, v
+  float m[PBX_PS_HEADS][PBX_HA_WAVES], l[PBX_PS_HEADS][PBX_HA_WAVES];
+  float acc[PBX_PS_HEADS][PBX_HA_WAVES][PBX_HA_MAX_HD];
+  unsigned absent[PBX_HA_WAVES];  // bits of the parts whose state a wave missed
+};
+
+// The states w and w + 8 of a head that wave w holds: maximum, sum, the lane's
+// dim of the V sum.
+struct SplitStates {
+  float m[2], l[2], a[2];
+};
+
+// The wave's two states merged into st_m / st_l / st_acc.
+__device__ __forceinline__ void split_store(const SplitStates &s, const int w, const int lane,
+                                            float *st_m, float *st_l,
+                                            float (*st_acc)[PBX_HA_MAX_HD]) {
+  const float mw = fmaxf(s.m[0], s.m[1]);
+  float lw = 0.f, aw = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float e = s.m[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s.m[i] - mw);
+    lw = fmaf(e, s.l[i], lw);
+    aw = fmaf(e, s.a[i], aw);
+  }
+  if (lane == 0) {
+    st_m[w] = mw;
+    st_l[w] = lw;
+  }
+  st_acc[w][lane] = aw;
+}
+
+// The 8 waves' states of one head, merged.
+__device__ __forceinline__ void split_merge(const float *pm, const float *pl,
+                                            const float (*pa)[PBX_HA_MAX_HD], const int lane,
+                                            float &M, float &den, float &num) {
+  M = -INFINITY, den = 0.f, num = 0.f;
+#pragma unroll
+  for (int i = 0; i < PBX_HA_WAVES; ++i) M = fmaxf(M, pm[i]);
+#pragma unroll
+  for (int i = 0; i < PBX_HA_WAVES; ++i) {
+    const float mi = pm[i];
+    const float e = mi == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mi - M);
+    den = fmaf(e, pl[i], den);
+    num = fmaf(e, pa[i][lane], num);
+  }
+}
+
+// Leaves the states of query head h in s and st_m / st_l / st_acc (wave w holds
+// the states w and w + 8 of the head's 4 * parts <= 16) and in absent[w] the
+// bits of those that did not arrive, for the barrier that follows.
 __device__ __forceinline__ void attention_split_states(const AttnArgs &a, const int h,
                                                        const int part, const int parts,
                                                        const int nc, const unsigned tag,
+                                                       SplitStates &s, SplitLds &sh,
                                                        float *st_m, float *st_l,
                                                        float (*st_acc)[PBX_HA_MAX_HD]) {
   constexpr int HG = PBX_PS_HEADS, HD = PBX_HA_MAX_HD, NW = PBX_HA_WAVES;
-  __shared__ __attribute__((aligned(16))) float rows[HG + 2][HD];  // q of the heads, new k, v
-  __shared__ float ps_m[HG][NW], ps_l[HG][NW];
-  __shared__ __attribute__((aligned(16))) float ps_acc[HG][NW][HD];
+  auto &rows = sh.rows;
+  auto &ps_m = sh.m, &ps_l = sh.l;
+  auto &ps_acc = sh.acc;
   const int Gq = a.n_heads / a.n_kv_heads, g = h / Gq, kvdim = a.n_kv_heads * HD;
   const int h0 = h - h % HG, p = h % HG + HG * part, P = HG * parts;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -864,6 +924,8 @@ __device__ __forceinline__ void attention_split_states(const AttnArgs &a, const 
   const float *kb = a.kcache + (size_t)g * HD, *vb = a.vcache + (size_t)g * HD;
   const int spin = a.spin > 0 ? a.spin : PBX_CELL_SPIN;
   const unsigned ptag = tag - (unsigned)a.skew;  // published with the launch's own tag
+  const int pspin = a.pspin > 0 ? a.pspin : PBX_PEER_SPIN;
+  const unsigned want = ptag + (unsigned)a.pskew;
 
   float m[HG], l[HG];
   float4 acc[HG], qq[HG], kn = make_float4(0.f, 0.f, 0.f, 0.f), vn = kn;
@@ -932,16 +994,8 @@ __device__ __forceinline__ void attention_split_states(const AttnArgs &a, const 
   }
   lds_barrier();
   if (w < HG) {
-    float M = -INFINITY, den = 0.f, num = 0.f;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) M = fmaxf(M, ps_m[w][i]);
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      const float mi = ps_m[w][i];
-      const float e = mi == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mi - M);
-      den = fmaf(e, ps_l[w][i], den);
-      num = fmaf(e, ps_acc[w][i][lane], num);
-    }
+    float M, den, num;
+    split_merge(ps_m[w], ps_l[w], ps_acc[w], lane, M, den, num);
     unsigned long long *cp = a.pcells + ((size_t)(h0 + w) * P + p) * PBX_PS_CELLS;
     const unsigned long long th = (unsigned long long)ptag << 32;
     __hip_atomic_store(cp + lane, th | __float_as_uint(num), __ATOMIC_RELAXED,
@@ -966,44 +1020,133 @@ __device__ __forceinline__ void attention_split_states(const AttnArgs &a, const 
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     v[i] = use[i] ? __hip_atomic_load(cp[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                  : (unsigned long long)ptag << 32;
+                  : (unsigned long long)want << 32;
   auto missing = [&]() {
-    return (unsigned)(v[0] >> 32) != ptag || (unsigned)(v[1] >> 32) != ptag ||
-           (unsigned)(v[2] >> 32) != ptag || (unsigned)(v[3] >> 32) != ptag;
+    return (unsigned)(v[0] >> 32) != want || (unsigned)(v[1] >> 32) != want ||
+           (unsigned)(v[2] >> 32) != want || (unsigned)(v[3] >> 32) != want;
   };
-  for (int it = 0; missing() && it < spin; ++it) {
+  for (int it = 0; missing() && it < pspin; ++it) {
     __builtin_amdgcn_s_sleep(1);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if ((unsigned)(v[i] >> 32) != ptag)
+      if ((unsigned)(v[i] >> 32) != want)
         v[i] = __hip_atomic_load(cp[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (missing())
-    __hip_atomic_fetch_or(a.status, PBX_DEV_WAIT_TIMEOUT, __ATOMIC_RELAXED,
-                          __HIP_MEMORY_SCOPE_AGENT);
-  float f[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    f[i] = (unsigned)(v[i] >> 32) == ptag ? __uint_as_float((unsigned)v[i]) : __builtin_nanf("");
-  float mw = -INFINITY, lw = 0.f, aw = 0.f, M[2], D[2];
+  unsigned gone = 0u;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    M[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[2 + i]), 0));
-    D[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[2 + i]), 1));
-    if (w + NW * i >= P) M[i] = -INFINITY;
-    mw = fmaxf(mw, M[i]);
+    const unsigned ml = (unsigned)v[2 + i];
+    s.m[i] = __uint_as_float(__builtin_amdgcn_readlane(ml, 0));
+    s.l[i] = __uint_as_float(__builtin_amdgcn_readlane(ml, 1));
+    s.a[i] = __uint_as_float((unsigned)v[i]);
+    if (w + NW * i >= P) s.m[i] = -INFINITY;
+    if (__any((unsigned)(v[i] >> 32) != want || (unsigned)(v[2 + i] >> 32) != want))
+      gone |= 1u << (w + NW * i);
   }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const float e = M[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M[i] - mw);
-    lw = fmaf(e, D[i], lw);
-    aw = fmaf(e, f[i], aw);
+  if (lane == 0) sh.absent[w] = gone;
+  split_store(s, w, lane, st_m, st_l, st_acc);
+}
+
+// The states of query head h over the parts `todo` (bits), whose workgroups'
+// own did not arrive: what split_chunk and the merges of
+// attention_split_states compute, the same operations in the same order, in a
+// loop over the slots (small code for a rare path; K is read twice).  The
+// waves meet in LDS; wave p % 8 gets the state of part p.
+__device__ __forceinline__ void split_absent(const AttnArgs &a, const int h, const int parts,
+                                             const int nc, const unsigned tag, unsigned todo,
+                                             SplitStates &s, SplitLds &sh, float *st_m,
+                                             float *st_l, float (*st_acc)[PBX_HA_MAX_HD]) {
+  constexpr int HD = PBX_HA_MAX_HD;
+  auto &row = sh.rows;
+  auto &fm = sh.m[0], &fl = sh.l[0];
+  auto &fa = sh.acc[0];
+  // recomputed here: kept from the caller, the lane's indices would cost the
+  // common paths registers
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63, w = tid >> 6, dcol = 4 * (lane & 15), pl = 4 * w + (lane >> 4);
+  const int g = h / (a.n_heads / a.n_kv_heads), kvdim = a.n_kv_heads * HD;
+  const int P = PBX_PS_HEADS * parts, ns = (nc + 31) / 32;
+  const float *kb = a.kcache + (size_t)g * HD, *vb = a.vcache + (size_t)g * HD;
+  if (w < 3)  // wave 0: q of head h; 1, 2: the newest k, v of KV head g
+    row[w][lane] = poll_cell(
+        a.cells + (w == 0 ? h * HD : a.qdim + (w - 1) * kvdim + g * HD) + lane, tag,
+        a.spin > 0 ? a.spin : PBX_CELL_SPIN, a.status);
+  lds_barrier();
+  const float c = a.scale * 1.44269504088896340736f;  // scale * log2 e
+  const float4 q4 = *reinterpret_cast<const float4 *>(&row[0][dcol]);
+  const float4 kn = *reinterpret_cast<const float4 *>(&row[1][dcol]);
+  const float4 vn = *reinterpret_cast<const float4 *>(&row[2][dcol]);
+  const float4 qq = make_float4(q4.x * c, q4.y * c, q4.z * c, q4.w * c);
+  auto cached = [&](const float *b, const float4 newest, int pos) -> float4 {
+    float4 t = *reinterpret_cast<const float4 *>(b + (size_t)min(pos, nc - 1) * kvdim + dcol);
+    if (pos >= nc - 1) t = newest;
+    return t;
+  };
+  auto score = [&](int pos) -> float {
+    const float4 k = cached(kb, kn, pos);
+    const float d = wave_sum<8>(fmaf(qq.x, k.x, fmaf(qq.y, k.y, fmaf(qq.z, k.z, qq.w * k.w))));
+    return pos < nc ? d : -INFINITY;
+  };
+#pragma unroll 1
+  for (; todo; todo &= todo - 1u) {
+    const int p = __builtin_ctz(todo);
+    float m = -INFINITY, l = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 1
+    for (int s0 = p; s0 < ns;) {
+      const int J = min(PBX_PS_SLOTS, (ns - s0 + P - 1) / P);
+      float mc = -INFINITY;
+#pragma unroll 1
+      for (int j = 0; j < J; ++j) mc = fmaxf(mc, score(32 * (s0 + P * j) + pl));
+      const float mn = fmaxf(m, mc);
+      const float ms = mn == -INFINITY ? 0.f : mn;  // a row with no position yet
+      const float f = __builtin_amdgcn_exp2f(m - ms);
+      float ls = 0.f;
+      float4 t = make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
+#pragma unroll 1
+      for (int j = 0; j < J; ++j) {
+        const int pos = 32 * (s0 + P * j) + pl;
+        const float e = __builtin_amdgcn_exp2f(score(pos) - ms);
+        const float4 v = cached(vb, vn, pos);
+        ls += e;
+        t.x = fmaf(e, v.x, t.x);
+        t.y = fmaf(e, v.y, t.y);
+        t.z = fmaf(e, v.z, t.z);
+        t.w = fmaf(e, v.w, t.w);
+      }
+      l = fmaf(l, f, ls);
+      acc = t;
+      m = mn;
+      s0 += J * P;
+    }
+    const float mw = pair_max<32>(pair_max<16>(m));
+    const float er = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mw);
+    const float lw = pair_sum<32>(pair_sum<16>(l * er));
+    const float4 aw = make_float4(pair_sum<32>(pair_sum<16>(acc.x * er)),
+                                  pair_sum<32>(pair_sum<16>(acc.y * er)),
+                                  pair_sum<32>(pair_sum<16>(acc.z * er)),
+                                  pair_sum<32>(pair_sum<16>(acc.w * er)));
+    if (lane == 0) {
+      fm[w] = mw;
+      fl[w] = lw;
+    }
+    if (lane < 16) *reinterpret_cast<float4 *>(&fa[w][dcol]) = aw;
+    lds_barrier();
+    if (w == (p & (PBX_HA_WAVES - 1))) {
+      float M, den, num;
+      split_merge(fm, fl, fa, lane, M, den, num);
+      const bool hi = p >= PBX_HA_WAVES;
+      s.m[0] = hi ? s.m[0] : M;
+      s.l[0] = hi ? s.l[0] : den;
+      s.a[0] = hi ? s.a[0] : num;
+      s.m[1] = hi ? M : s.m[1];
+      s.l[1] = hi ? den : s.l[1];
+      s.a[1] = hi ? num : s.a[1];
+    }
+    lds_barrier();  // before fm, fl and fa are used again
   }
-  if (lane == 0) {
-    st_m[w] = mw;
-    st_l[w] = lw;
-  }
-  st_acc[w][lane] = aw;
+  split_store(s, w, lane, st_m, st_l, st_acc);
 }
 
 // MAXJ: position slots a wave keeps in flight (16 slots of K and V are
@@ -1064,11 +1207,18 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
   int s0 = 0;
   unsigned tag = 0;
   bool split = false;
+  SplitStates sst;
+  __shared__ __attribute__((aligned(16))) SplitLds sh;
   if constexpr (FUSED) {
     tag = cell_tag(a.epoch ? *a.epoch : a.cells[a.cell_n]) + (unsigned)a.skew;
     const int spin = a.spin > 0 ? a.spin : PBX_CELL_SPIN;
     float4 kn = make_float4(0.f, 0.f, 0.f, 0.f), vn = kn;
+    bool first = true;
+    // (one instance of a chunk size, first or not: code that a launch has not
+    // run yet comes from L2 line by line, and the second chunk of 600 positions
+    // in an instance of its own took 366 us a token against 351)
     auto ready = [&]() {
+      if (!first) return;
       if (w < 3) {  // wave 0: q of head h; 1, 2: k, v of KV head g
         nrow[w][lane] =
             lane < hd ? poll_cell(a.cells + (w == 0 ? h * hd : a.qdim + (w - 1) * kvdim + g * hd) +
@@ -1084,8 +1234,6 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
       kn = *reinterpret_cast<const float4 *>(&nrow[1][dcol]);
       vn = *reinterpret_cast<const float4 *>(&nrow[2][dcol]);
     };
-    auto none = [] {};
-    bool first = true;
     if constexpr (IPT > 0) split = a.split_at > 0 && nc > a.split_at;
     while (!split && 32 * s0 < nc) {
       const int J = min(MAXJ, (nc - 32 * s0 + 31) / 32);
@@ -1093,10 +1241,7 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
 #define PBX_HEAD_CHUNK_N(n)                                                                \
   case n:                                                                                  \
     if constexpr (n <= MAXJ) {                                                             \
-      if (first)                                                                           \
         head_chunk_n<n>(kb, vb, kvdim, dcol, s0, pl, nc, ready, qq, kn, vn, m, l, acc);    \
-      else                                                                                 \
-        head_chunk_n<n>(kb, vb, kvdim, dcol, s0, pl, nc, none, qq, kn, vn, m, l, acc);     \
     }                                                                                      \
     break;
         PBX_HEAD_CHUNK_N(1) PBX_HEAD_CHUNK_N(2) PBX_HEAD_CHUNK_N(3) PBX_HEAD_CHUNK_N(4)
@@ -1129,8 +1274,10 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
   }
 
   if constexpr (FUSED && IPT > 0) {
-    if (split)
-      attention_split_states(a, h, part, a.n_heads * hd / (256 * IPT), nc, tag, st_m, st_l, st_acc);
+    if (split) {
+      const int parts = a.n_heads * hd / (256 * IPT);
+      attention_split_states(a, h, part, parts, nc, tag, sst, sh, st_m, st_l, st_acc);
+    }
   }
   if (!split) {
     // merge in two levels: the wave's 4 rows (same dims, 16 lanes apart) in
@@ -1149,6 +1296,19 @@ __device__ __forceinline__ void attention_cached_body(const AttnArgs &a, const i
     if (lane < 16) *reinterpret_cast<float4 *>(&st_acc[w][4 * dg]) = aw;
   }
   lds_barrier();
+  if constexpr (FUSED && IPT > 0) {
+    if (split) {
+      unsigned todo = 0u;
+#pragma unroll
+      for (int i = 0; i < PBX_HA_WAVES; ++i) todo |= sh.absent[i];
+      todo = __builtin_amdgcn_readfirstlane(todo);
+      if (__builtin_expect(todo != 0u, 0)) {
+        split_absent(a, h, a.n_heads * hd / (256 * IPT), nc, tag, todo, sst, sh, st_m,
+                     st_l, st_acc);
+        lds_barrier();
+      }
+    }
+  }
   if (w == 0) {
     const float mi = lane < PBX_HA_WAVES ? st_m[lane] : -INFINITY;
     const float li = lane < PBX_HA_WAVES ? st_l[lane] : 0.f;

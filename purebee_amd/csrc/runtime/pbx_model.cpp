@@ -50,9 +50,12 @@ struct AttnArgsHost {  // AttnArgs in pbx_decode.hip
   const unsigned long long *epoch = nullptr;
   unsigned long long *ocells = nullptr;
   // pbx_qkvr_attn_o_*: cells of the partial states and the context length
-  // above which the positions are split over a KV group's workgroups
+  // above which the positions are split over a KV group's workgroups; the
+  // test-only tag offset of the peers' states and their poll limit (0: the
+  // kernel's default)
   unsigned long long *pcells = nullptr;
   int split_at = 0;
+  int pskew = 0, pspin = 0;
 };
 
 struct AttnSplitArgsHost {  // AttnSplitArgs in pbx_decode.hip
@@ -241,6 +244,9 @@ struct pbx_model {
   // pbx_model_test_handoff: the fused launch of layer test_layer waits for
   // tags offset by test_skew, with at most test_spin polls (0: default)
   int test_layer = -1, test_skew = 0, test_spin = 0;
+  // pbx_model_test_peers: every joined launch that splits its context expects
+  // its peers' states under tags offset by test_pskew
+  int test_pskew = 0, test_pspin = 0;
   int *hist = nullptr;
   int hist_cap = 0;
   std::vector<Op> ops;
@@ -716,8 +722,9 @@ static int build_ops(pbx_model *m) {
   const std::string qa_name = o_ipt == 2 ? "pbx_qkvr_attn_o_r8c2" : "pbx_qkvr_attn_o_r4c1";
   if ((o_ipt == 1 || o_ipt == 2) && qa_fit) fqa = pbx_kernel_by_name(c, qa_name);
   // Long contexts: the positions split over the 16 workgroups of four heads
-  // of a KV group, which wait for each other's states, so the whole grid (one
-  // workgroup a CU) must fit the CUs.
+  // of a KV group, which wait a short time for each other's states and then
+  // compute the absent ones themselves.  Worth it only where a group usually
+  // runs at once: the whole grid (one workgroup a CU) fits the CUs.
   const int parts = o_ipt ? g.dim / (256 * o_ipt) : 0;
   const bool qa_split = fqa && m->attn_split > 0 && g.n_heads / g.n_kv_heads % 4 == 0 &&
                         4 * parts <= 16 &&
@@ -815,6 +822,8 @@ static int build_ops(pbx_model *m) {
         if (qa_split) {
           a.attn.pcells = cells + m->qkv_rows + 64;
           a.attn.split_at = m->attn_split;
+          a.attn.pskew = m->test_pskew;
+          a.attn.pspin = m->test_pspin;
         }
         if (l == m->test_layer) {
           a.attn.skew = m->test_skew;
@@ -2404,6 +2413,15 @@ extern "C" int pbx_model_op_name(const pbx_model *m, int i, char *buf, size_t ca
   return PBX_OK;
 }
 
+// New kernel arguments for a test: the step's launches and every captured
+// graph are made again.
+static int rebuild_ops(pbx_model *m) {
+  drop_graph(m);
+  m->ops_ready = false;
+  const int rc = check_complete(m);
+  return rc ? rc : build_ops(m);
+}
+
 extern "C" int pbx_model_test_handoff(pbx_model *m, int layer, int skew, int spin) {
   if (!model_ok(m)) return pbx_fail(nullptr, PBX_EINVAL, "pbx_model_test_handoff: not a live model");
   if (layer >= m->cfg.n_layers || spin < 0)
@@ -2412,16 +2430,27 @@ extern "C" int pbx_model_test_handoff(pbx_model *m, int layer, int skew, int spi
   m->test_layer = layer;
   m->test_skew = skew;
   m->test_spin = spin;
-  // the kernels' arguments change: rebuild them and every captured graph
-  drop_graph(m);
-  m->ops_ready = false;
-  int rc = check_complete(m);
-  if (rc || (rc = build_ops(m))) return rc;
+  int rc = rebuild_ops(m);
+  if (rc) return rc;
   for (const Op &op : m->ops)
     if (op.kind == ARG_FUSED || op.kind == ARG_SMALL) return PBX_OK;
   return layer < 0 ? PBX_OK
                    : pbx_fail(m->c, PBX_ENOTSUP,
                               "pbx_model_test_handoff: the step has no joined q|k|v + attention launch");
+}
+
+extern "C" int pbx_model_test_peers(pbx_model *m, int skew, int spin) {
+  if (!model_ok(m)) return pbx_fail(nullptr, PBX_EINVAL, "pbx_model_test_peers: not a live model");
+  if (spin < 0)
+    return pbx_fail(m->c, PBX_EINVAL, "pbx_model_test_peers: spin %d out of range", spin);
+  m->test_pskew = skew;
+  m->test_pspin = spin;
+  int rc = rebuild_ops(m);
+  if (rc) return rc;
+  for (const Op &op : m->ops)
+    if (op.kind == ARG_FUSED && op.attn.split_at > 0) return PBX_OK;
+  return pbx_fail(m->c, PBX_ENOTSUP,
+                  "pbx_model_test_peers: the step has no launch that splits long contexts");
 }
 
 extern "C" int pbx_model_bench_role(pbx_model *m, const char *role, int reps,

@@ -40,6 +40,7 @@ EXPORTS = (
     "pbx_model_create", "pbx_model_free", "pbx_model_set_tensor", "pbx_model_forward",
     "pbx_model_forward_batch", "pbx_model_generate", "pbx_model_generate_eos", "pbx_model_reset_cache", "pbx_model_rollback", "pbx_model_info",
     "pbx_model_profile", "pbx_model_op_name", "pbx_model_bench_role", "pbx_model_test_handoff",
+    "pbx_model_test_peers",
     "pbx_speculative_generate", "pbx_model_forward_layers", "pbx_self_speculative_generate",
     "pbx_gguf_open", "pbx_gguf_close", "pbx_gguf_info", "pbx_gguf_tensor_info",
     "pbx_gguf_find_tensor", "pbx_gguf_get_int", "pbx_gguf_get_float", "pbx_gguf_get_string",
@@ -174,6 +175,7 @@ def load_library():
         "pbx_model_reset_cache": (ctypes.c_int, [_vp]),
         "pbx_model_rollback": (ctypes.c_int, [_vp, ctypes.c_int]),
         "pbx_model_test_handoff": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+        "pbx_model_test_peers": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int]),
         "pbx_model_info": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_size_t),
                                           ctypes.POINTER(ctypes.c_int)]),
         "pbx_model_profile": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int, ctypes.c_int,
@@ -582,6 +584,12 @@ class Model:
         for cells that never arrive (tag offset `skew`), giving up after
         `spin` polls; layer < 0 restores the normal launch."""
         self._mcall("pbx_model_test_handoff", layer, skew, spin)
+
+    def test_peers(self, skew, spin=0):
+        """Test hook: the launches that split a long context wait for peers'
+        states that never arrive (tag offset `skew`, `spin` polls) and compute
+        them themselves; skew 0 restores the normal launch."""
+        self._mcall("pbx_model_test_peers", skew, spin)
 
     def info(self):
         b, g = ctypes.c_size_t(), ctypes.c_int()

@@ -308,6 +308,81 @@ def test_split_context_attention(ctx, default_paths, kv_heads, n):
     assert all(np.isfinite(a).all() for a in out["1"][0])
     assert worst <= 1e-4
     assert out["0"][1] == out["1"][1]
+    if n >= 510:  # another order of sums: equal bits would mean that nothing was split
+        assert not any(np.array_equal(a, b) for a, b in zip(out["0"][0], out["1"][0]))
+
+
+def split_model(ctx, seed, **kw):
+    cfg = tiny(TYPE_Q4_0, TYPE_Q4_0, dim=2048, hidden_dim=8192, n_layers=2, n_heads=32,
+               n_kv_heads=8, vocab_size=512, max_seq=4128)
+    cfg.update(kw)
+    return synth.build(ctx, cfg, seed), [int(t) for t in synth.random_tokens(seed + 1, 4128, 512)]
+
+
+@pytest.mark.parametrize("kv_heads", [8, 4])
+@pytest.mark.parametrize("n", [1, 40, 700, 4094])
+def test_split_context_absent_peers(ctx, default_paths, kv_heads, n):
+    """The split context when no peer's state ever arrives (the test hook
+    offsets the tag expected of the peers' cells; 3 polls): every workgroup
+    computes the absent states itself, by the peers' own code and order, so
+    the call succeeds and its logits and greedy tokens are the normal launch's
+    bit for bit; from one slot of positions (all other parts are empty) to
+    two chunks of slots a part."""
+    print(f"[case] absent peers, {kv_heads} KV heads, position {n}..", flush=True)
+    default_paths.setenv("PBX_ATTN_SPLIT", "1")
+    model, toks = split_model(ctx, 151, n_kv_heads=kv_heads)
+    model.forward(toks[:n], 0, want_logits=False)
+    out = []
+    for skew in (0, 1, 0):
+        model.test_peers(skew, 3 if skew else 0)
+        out.append([model.forward([toks[n + i]], n + i)[0] for i in range(2)])
+        out[-1].append(model.generate(toks[n], n, 20))
+    model.free()
+    assert all(np.isfinite(a).all() for a in out[0])
+    for other in out[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(out[0], other))
+
+
+def test_split_context_concurrent_streams(ctx, default_paths):
+    """Three models, each with its own context and thread, decode split
+    contexts at once: their launches share the CUs, so a group of workgroups
+    need not run as a whole.  Every call succeeds, with the tokens and logits
+    of the same model alone, bit for bit.  (The joined FFN, whose slices do
+    wait for each other, is off.)"""
+    import threading
+    import purebee_amd as pb
+    print("[case] three streams decode split contexts", flush=True)
+    default_paths.setenv("PBX_FFN", "0")
+    default_paths.setenv("PBX_ATTN_SPLIT", "1")
+    n, steps = 900, 24
+    ctxs = [pb.Context(0) for _ in range(3)]
+    models = [split_model(c, 161 + 10 * i) for i, c in enumerate(ctxs)]
+    alone = []
+    for model, toks in models:
+        model.forward(toks[:n], 0, want_logits=False)
+        alone.append(model.generate(toks[n], n, steps, want_logits=True))
+    got = [None] * 3
+
+    def work(i):
+        model, toks = models[i]
+        try:
+            got[i] = [model.generate(toks[n], n, steps, want_logits=True) for _ in range(4)]
+        except Exception as e:  # reported below, on the main thread
+            got[i] = e
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in range(3):
+        assert isinstance(got[i], list), got[i]
+        for toks, logits in got[i]:
+            assert list(toks) == list(alone[i][0]) and np.array_equal(logits, alone[i][1])
+    for model, _ in models:
+        model.free()
+    for c in ctxs:
+        c.close()
 
 
 def test_non_finite_activation_propagates(ctx):
