@@ -421,6 +421,68 @@ ROWS_KERNELS(f16, PBX_F16)
 ROWS_KERNELS(q6k, PBX_Q6K)
 
 // ---------------------------------------------------------------------------
+// Few rows of long K into a narrow matrix (pbx_gemm_<type>_p16): 5 to 16 rows
+// whose 16-row tiles of W leave at least half of the CUs idle.  There the
+// kernel above converts the rows' whole K in every workgroup, 6.4 us for each
+// 2048 columns of 16 rows; here the rows are prepared once (X16 / X16lo, Mpad =
+// 16) and K is split over blockIdx.z, for two launches more.  Q4_0 2048 x 8192
+// at 16 rows 18.5 us against 27.3, 64 x 16384 32.6 against 49.5 (bound by the
+// three launches and the latency of a split's loads).
+// Workgroup = 4 waves side by side along n, 16 x 16 outputs a wave, written as
+// a partial; the loop's steps are 8 blocks, all loaded before the first MFMA.
+// ---------------------------------------------------------------------------
+template <int TYPE>
+__device__ __forceinline__ void gemm_part16(const GemmArgs &a) {
+  constexpr int U = 8;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int li = lane & 15, g = lane >> 4;
+  const int n = (blockIdx.x * 4 + wave) * 16 + li, nr = min(n, a.Npad - 1);
+  const int per = (a.B + a.KS - 1) / a.KS;
+  const int b0 = blockIdx.z * per;
+  const int b1 = min(a.B, b0 + per);
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  floatx4 acc = zero;
+  for (int b = b0; b < b1; b += U) {
+    typename RawT<TYPE>::type raw[U];
+    unsigned dbits[U], mbits[U];
+    half8 A[U], Alo[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const int bb = min(b + j, b1 - 1);
+      const size_t blk = (size_t)nr * a.B + bb;
+      if constexpr (TYPE == PBX_F16)
+        raw[j] = *reinterpret_cast<const uint4 *>(a.qs + (blk * 32 + 8 * g) * 2);
+      else if constexpr (TYPE == PBX_Q8)
+        raw[j] = *reinterpret_cast<const uint2 *>(a.qs + blk * 32 + g * 8);
+      else
+        raw[j] = *reinterpret_cast<const uint2 *>(a.qs + blk * 16 + (g & 1) * 8);
+      dbits[j] = TYPE == PBX_F16 ? 0x3C00u : a.dsc[dsc_index(nr, bb, a.B)];
+      mbits[j] = TYPE == PBX_Q41 ? a.msc[dsc_index(nr, bb, a.B)] : 0u;
+      const size_t off = ((size_t)bb * 16 + li) * 32 + 8 * g;
+      A[j] = *reinterpret_cast<const half8 *>(a.X16 + off);
+      Alo[j] = *reinterpret_cast<const half8 *>(a.X16lo + off);
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      if (b + j < b1)
+        block_mma<TYPE>(acc, A[j], Alo[j], codes_operand<TYPE>(raw[j], g),
+                        f16_bits_to_f32(dbits[j]), f16_bits_to_f32(mbits[j]),
+                        TYPE == PBX_Q41 ? block_sums(A[j], Alo[j]) : zero);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int m = 4 * g + r;
+    if (m < a.M && n < a.N) a.Y[((size_t)blockIdx.z * a.M + m) * a.N + n] = acc[r] * a.inv[m];
+  }
+}
+
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q4_p16(GemmArgs a) { gemm_part16<PBX_Q4>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q8_p16(GemmArgs a) { gemm_part16<PBX_Q8>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_q41_p16(GemmArgs a) { gemm_part16<PBX_Q41>(a); }
+extern "C" __global__ void __launch_bounds__(256) pbx_gemm_f16_p16(GemmArgs a) { gemm_part16<PBX_F16>(a); }
+
+// ---------------------------------------------------------------------------
 // Large-M kernel (M > 32): 32x32x16 MFMAs with every operand moved to LDS
 // by DMA.  Operand lane layout of v_mfma_f32_32x32x16_f16 (checked on
 // the device): A: lane l holds A[l%32][8*(l/32) + e]; B: lane l holds

@@ -181,6 +181,34 @@ int launch_rows(pbx_ctx *c, const pbx_weight *w, const float *dX, int M, const f
                        dim3(64 * std::min(8, chunks)), args, stream);
 }
 
+// Up to PBX_GEMM_ROWS_M rows, where the one-launch kernel loses because every
+// workgroup converts its rows' whole K (about 3.2 us a 1024 columns of 16
+// rows, however few the workgroups):
+// * few columns and long rows: pbx_gemm_<type>_p16, K split over workgroups.
+//   Q4_0 2048 x 8192: 16 rows 18.5 us against 27.3, 12 rows 18.3 / 23.3, 8 rows
+//   18.2 / 20.5; 2048 x 6144, 11 rows 15.7 / 18.6; 2048 x 4096, 16 rows 12.9 /
+//   15.4; so from 64 K activation values on.  Q4_1, whose block sums cost the
+//   one-launch kernel more, from 48 K (2048 x 8192, 8 rows 19.7 / 24.0).  Not
+//   for 4 rows (F16 2048 x 16384 33 / 30), nor past half the CUs' tiles.
+bool few_columns(const pbx_ctx *c, const pbx_weight *w, int M) {
+  const int64_t values = (int64_t)M * w->B * 32;
+  return M > 4 && M <= 16 && (w->N + 15) / 16 <= c->cu_count / 2 &&
+         values >= (w->type == PBX_TYPE_Q4_1 ? 48 << 10 : 64 << 10);
+}
+// * many rounds of 32 x 32 tiles of more than 2048 columns (shorter rows stay
+//   in registers over the rounds): the prepared LDS-DMA GEMM.  Q4_0 32 rows
+//   16384 x 4096 50.4 us against 57.1, 32768 x 2304 48 / 68, 32768 x 8192 170 /
+//   210; 20 rows 16384 x 8192 90 / 88, 32768 x 4096 80 / 90; 32 rows 16384 x
+//   2304 35.1 / 34.6, Q8_0 38 / 34.5.  A weight beyond
+//   the 256 MB of the last-level cache comes from HBM either way, and the
+//   one-launch kernel streams it better (F16 32768 x 8192, 32 rows 248 / 206).
+bool many_columns(const pbx_ctx *c, const pbx_weight *w, int M) {
+  const int64_t tiles = (w->N + 31) / 32;
+  return M > 16 && w->B > 64 && M * tiles >= 64 * (int64_t)c->cu_count &&
+         M * tiles * w->B >= 5120 * (int64_t)c->cu_count &&
+         w->N * pbx_type_row_bytes(w->type, w->K) <= 256 << 20;
+}
+
 // Workspace of the prepared GEMM: the fp16 pair, the row scales and the
 // split-K partials.
 struct GemmSpace {
@@ -265,17 +293,29 @@ int pbx_gemm_launch(pbx_ctx *c, const pbx_weight *w, const float *dX, int64_t M6
     return launch_rows(c, w, dX, (int)M64, dBias, dY, accumulate, stream);
   }
   const int M = (int)M64, N = (int)w->N, K = (int)w->B * 32;
-  if (M <= PBX_GEMM_ROWS_M) {
-    // (no workspace needed; a caller's limits K as it does for more rows)
+  pbx_gemm_plan p;
+  int rc;
+  if (few_columns(c, w, M)) {
+    p.M = M;
+    p.Mpad = 16;
+    p.mtiles = 1;
+    p.nwg = (N + 63) / 64;
+    p.KS = 8;  // at least 16 times the tiles would fill the CUs; K is long
+    p.name = std::string("pbx_gemm_") + gemm_tag(w->type) + "_p16";
+  } else if ((M > PBX_GEMM_ROWS_M || many_columns(c, w, M)) &&
+             (rc = pbx_gemm_make_plan(c, w, M, &p))) {
+    return rc;
+  }
+  GemmSpace sp = gemm_space(p, N, K);
+  if (!p.M || (M <= PBX_GEMM_ROWS_M && wsp && sp.total() > wsp->bytes)) {
+    // One launch on the fp32 rows: no workspace is used.  A caller that brings
+    // one is still refused a K whose fp16 pair it could not hold: this entry's
+    // limit has always been that, whichever kernel a shape takes.
     char *unused = nullptr;
     const size_t pair = (size_t)(M <= 16 ? 16 : 32) * K * 4;
-    int rc = wsp ? workspace(c, wsp, pair, &unused) : PBX_OK;
+    rc = wsp ? workspace(c, wsp, pair, &unused) : PBX_OK;
     return rc ? rc : launch_rows(c, w, dX, M, dBias, dY, accumulate, stream);
   }
-  pbx_gemm_plan p;
-  int rc = pbx_gemm_make_plan(c, w, M, &p);
-  if (rc) return rc;
-  const GemmSpace sp = gemm_space(p, N, K);
   char *ws = nullptr;
   if ((rc = workspace(c, wsp, sp.total(), &ws))) return rc;
   // fp16 activations and their fp16 rounding residuals

@@ -541,9 +541,20 @@ int pbx_linear_enqueue(pbx_ctx *c, const pbx_weight *w, const float *dX, int64_t
     return pbx_launch(c, PBX_K_GEMV_Q8REF, dim3((unsigned)((N + 63) / 64), gy), dim3(512),
                       args, stream);
   }
-  if (M >= PBX_GEMM_MIN_M)
-    return pbx_gemm_enqueue(c, w, dX, M, dBias, dY, stream, ws);
   int B = (int)w->B;
+  // Q6_K: a GEMV pass per row while the call is small, since a workgroup of
+  // the GEMM converts its rows' whole K however few columns it has: 256 x 8192
+  // at 16 rows 9.9 us against 24.1, 1000 x 4096 at 4 rows 7.5 / 9.5, 2048 x 2048
+  // at 4 rows 6.2 / 6.5; above the line 1000 x 2048 at 16 rows 9.6 / 8.6, 2048 x
+  // 8192 at 4 rows 18.2 / 15.8.  Short K: 256 x 1024 at 16 rows 5.0 / 5.5, at 8
+  // rows 4.9 / 4.8; below 1024 the GEMM is never slower.
+  const int64_t outs = (int64_t)N * M;
+  const bool q6k_gemv =
+      w->type == PBX_TYPE_Q6_K &&
+      (B >= 64 ? outs <= (M <= 8 ? 8192 : 12288) - (B >= 256 ? 2048 : 0)
+               : B >= 32 && M > 8 && outs <= 8192);
+  if (M >= PBX_GEMM_MIN_M && !q6k_gemv)
+    return pbx_gemm_enqueue(c, w, dX, M, dBias, dY, stream, ws);
   // Integer-limb kernels (gemv_int) for Q4_0 / Q8_0 with K = 2048..8192 (not
   // 4097..6144): rows per workgroup by N so the grid keeps >= 256 workgroups
   // where it can, and the tile loop (two workgroups a CU) for tall matrices

@@ -122,3 +122,40 @@ def test_tiny_rows_stay_finite(ctx, t, M, K):
     assert np.isfinite(Y).all() and not Y[2].any()
     for m in (0, 1, M - 1):
         assert error(Y[m], oracle.matvec(t, X[m], raw, N, K), X[m]) <= 1e-5
+
+
+@pytest.mark.parametrize("t", TYPES[:4])
+@pytest.mark.parametrize("M,N,K", [(16, 1, 6144), (16, 70, 6176), (12, 2040, 8224), (9, 130, 12320),
+                                   (8, 100, 8192), (5, 33, 20000), (16, 2048, 6144)])
+def test_few_columns_long_rows(ctx, t, M, N, K):
+    """K split over workgroups (pbx_gemm_<type>_p16): its tile edges in N, row
+    counts short of the tile, K that the 8 splits and the steps of 8 blocks
+    do not divide."""
+    check(ctx, t, M, N, K, [0, 1, 2, 3, M - 1])
+
+
+@pytest.mark.parametrize("t", TYPES[:4])
+def test_many_columns_take_the_prepared_gemm(ctx, t):
+    check(ctx, t, 32, 16390, 2592, [0, 1, 2, 3, 31])
+
+
+@pytest.mark.parametrize("M,N,K", [(4, 48, 8192), (8, 1024, 2048), (16, 768, 2304), (100, 48, 1024),
+                                   (8, 1025, 2048), (16, 770, 2304), (9, 911, 1024)])
+def test_q6_k_both_sides_of_the_gemv_line(ctx, M, N, K):
+    check(ctx, pb.TYPE_Q6_K, M, N, K, [0, 1, 2, 3, M - 1])
+
+
+def test_q6_k_non_finite_rows_as_one_row(ctx):
+    """An infinite or NaN activation gives a Q6_K output row the NaNs that the
+    one-row GEMV gives it (every code is taken against an offset, so infinity
+    meets infinity of the other sign), through the GEMM as well."""
+    M, N, K = 6, 1400, 2048
+    w = ctx.upload(pb.TYPE_Q6_K, N, K, raw_weights(pb.TYPE_Q6_K, 9, N, K))
+    X = pb.synth_normal(10, M * K).reshape(M, K)
+    X[1, 7], X[2, 300], X[4, 2047] = np.inf, -np.inf, np.nan
+    Y = ctx.linear(w, X)
+    for m in range(M):
+        one = ctx.linear(w, X[m])
+        assert np.array_equal(np.isnan(one), np.isnan(Y[m]))
+        assert np.isnan(Y[m]).all() == (m in (1, 2, 4))
+    w.free()
