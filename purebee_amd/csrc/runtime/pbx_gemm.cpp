@@ -165,7 +165,8 @@ int launch_rows(pbx_ctx *c, const pbx_weight *w, const float *dX, int M, const f
   else if (wgs(1, 2) >= enough) NT = 2;
   // More than one round of workgroups: those of one a CU walk the tiles with
   // the activations in registers (K <= 2048).  16384 x 2048 Q8_0 at 20 rows
-  // 21.6 us against 28.6; 128256 x 2048 Q6_K at 5 rows 72 against 98.
+  // 21.6 us against 28.6; 128256 x 2048 Q6_K at 5 rows 72 against 98
+  // (in turn on one box; 80 on others).
   const bool loop = chunks <= 8 && NT > 1 && wgs(MT, NT) >= 2 * c->cu_count;
   if (loop) NT = MT == 1 ? 2 : 1;
   const std::string name = std::string("pbx_gemm_rows_") +
@@ -300,22 +301,22 @@ int pbx_gemm_launch(pbx_ctx *c, const pbx_weight *w, const float *dX, int64_t M6
     p.Mpad = 16;
     p.mtiles = 1;
     p.nwg = (N + 63) / 64;
-    p.KS = 8;  // at least 16 times the tiles would fill the CUs; K is long
+    p.KS = 8;  // the tiles alone are a wave each for at most half of the CUs
     p.name = std::string("pbx_gemm_") + gemm_tag(w->type) + "_p16";
   } else if ((M > PBX_GEMM_ROWS_M || many_columns(c, w, M)) &&
              (rc = pbx_gemm_make_plan(c, w, M, &p))) {
     return rc;
   }
-  GemmSpace sp = gemm_space(p, N, K);
-  if (!p.M || (M <= PBX_GEMM_ROWS_M && wsp && sp.total() > wsp->bytes)) {
+  if (!p.M) {
     // One launch on the fp32 rows: no workspace is used.  A caller that brings
-    // one is still refused a K whose fp16 pair it could not hold: this entry's
-    // limit has always been that, whichever kernel a shape takes.
+    // one is still refused a K whose fp16 pair it could not hold: its limit
+    // does not depend on the kernel that a shape takes.
     char *unused = nullptr;
     const size_t pair = (size_t)(M <= 16 ? 16 : 32) * K * 4;
     rc = wsp ? workspace(c, wsp, pair, &unused) : PBX_OK;
     return rc ? rc : launch_rows(c, w, dX, M, dBias, dY, accumulate, stream);
   }
+  const GemmSpace sp = gemm_space(p, N, K);
   char *ws = nullptr;
   if ((rc = workspace(c, wsp, sp.total(), &ws))) return rc;
   // fp16 activations and their fp16 rounding residuals

@@ -159,3 +159,19 @@ def test_q6_k_non_finite_rows_as_one_row(ctx):
         assert np.array_equal(np.isnan(one), np.isnan(Y[m]))
         assert np.isnan(Y[m]).all() == (m in (1, 2, 4))
     w.free()
+
+
+@pytest.mark.parametrize("t,M,N,K", [(pb.TYPE_Q4_0, 16, 70, 6176), (pb.TYPE_Q4_1, 7, 70, 8192),
+                                     (pb.TYPE_Q8_0, 32, 16390, 2592), (pb.TYPE_Q6_K, 4, 48, 2048)])
+def test_few_rows_noalloc_takes_the_same_kernels(ctx, t, M, N, K):
+    w = ctx.upload(t, N, K, raw_weights(t, M, N, K))
+    X = pb.synth_normal(N, M * K).reshape(M, K)
+    dx, dy = ctx.alloc(M * K * 4).upload(X), [ctx.alloc(M * N * 4) for _ in range(2)]
+    ctx.linear_dev(w, dx.ptr, M, dy[0].ptr)
+    ctx.linear_dev_noalloc(w, dx.ptr, M, dy[1].ptr)
+    ctx.sync()
+    a, b = (d.download(np.float32, M * N) for d in dy)
+    for d in (dx, *dy):
+        d.free()
+    w.free()
+    assert np.isfinite(a).all() and np.array_equal(a, b)
