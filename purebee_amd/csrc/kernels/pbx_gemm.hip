@@ -48,7 +48,7 @@ struct GemmArgs {
   int M, N, Npad, B, KS;
   int accumulate;         // 1: Y[m][n] += result (residual), single split only
   const uint16_t *msc;    // Q4_1 fp16 min plane
-  int Mpad;               // rows of a block of X16 (M padded to the kernel's M tile)
+  int Mpad;               // rows of a block of X16 (M padded to a multiple of 128; p16: 16)
 };
 
 namespace {
@@ -154,9 +154,11 @@ __device__ __forceinline__ floatx4 block_sums(half8 Ah, half8 Al) {
 // block is two products whose other half is zeroed.
 // Q4_0 8192 x 2048 at 16 rows: 12 us a call against 16.9 with preparation,
 // split GEMM and reduction as three launches (floor 2 us: one launch and the
-// latency of a chunk's loads are the rest); Q6_K 128256 x 2048 at 5 rows 72 us
-// against 350 with one GEMV pass a row (3.0 TB/s, the code unpacking beside the
-// loads bounds it).
+// latency of a chunk's loads are the rest); Q6_K 128256 x 2048 at 5 rows 80 us
+// against 350 with one GEMV pass a row (2.7 TB/s, the code unpacking beside the
+// loads bounds it).  The GEMV holds Q6_K's activations in all 24 bits but sums
+// 32 x beside the codes; the pair's errors are smaller (1.1e-7 against 3.7e-7,
+// also with outliers of 1e2 to 1e10 in a row).
 // ---------------------------------------------------------------------------
 #define ROWS_WV 8  // waves of a workgroup at most
 
