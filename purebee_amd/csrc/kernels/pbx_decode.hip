@@ -792,9 +792,9 @@ __device__ __forceinline__ float poll_cell(const unsigned long long *cp, unsigne
 // hardly ever run, costs every launch 0.2 us: 317 -> 320 us a token at KV 128,
 // 413 -> 416 at 3500.)
 // Bound by the K/V transfer and by the hand-off's ~2 us: Llama-1B decode at KV
-// 3500 888 -> 403 us a token, 2000: 543 -> 371, 1000: 406 -> 361.  The hand-off
-// costs more than it saves on short contexts (700: 374 unsplit against 363, 512:
-// 350 against 359, 128: 323 against 354), so split_at is 640.
+// 3500 730 us a token unsplit, 417 split, 1000: 388 / 363.  The hand-off costs
+// more than it saves on short contexts (800: 365.5 / 363, 750: 360.5 / 363, 600:
+// 351 / 363, 520: 346.5 / 363), so split_at is 768.
 #define PBX_PS_HEADS 4
 #define PBX_PS_CELLS 66  // 64 dims, maximum, sum
 #define PBX_PS_SLOTS 8   // slots in flight

@@ -237,7 +237,7 @@ struct pbx_model {
   unsigned long long *qa_cells = nullptr;
   // context length above which the joined launch splits the positions over
   // the workgroups of a KV group (PBX_ATTN_SPLIT at creation; 0: never)
-  int attn_split = 640;
+  int attn_split = 768;
   // state[0] position, [1] token, [2] step, [3] status word (bits set by
   // device-side waits that gave up; read and cleared by the host calls)
   int *state = nullptr;
